@@ -225,6 +225,27 @@ __global__ void __launch_bounds__(256) k_bert_attn(const float * __restrict__ qk
         op[i] = make_float4(O[4 * i] * inv, O[4 * i + 1] * inv, O[4 * i + 2] * inv, O[4 * i + 3] * inv);
 }
 
+// The features [rows][D] as the caller takes them, [D][len_b] per sequence, the sequences back to
+// back (src/gsv_bert.cpp:220-228): one 32 x 32 tile of a sequence per workgroup, through LDS.
+__global__ void __launch_bounds__(256) k_bert_features(const float * __restrict__ x,
+                                                       const int32_t * __restrict__ seq_off,
+                                                       const int32_t * __restrict__ seq_len, int D,
+                                                       float * __restrict__ out) {
+    const int b = blockIdx.z, d0 = blockIdx.y * 32, t0 = blockIdx.x * 32;
+    const int len = seq_len[b];
+    const int64_t off = seq_off[b];
+    if (t0 >= len) return;   // uniform over the workgroup
+    __shared__ float s[32][33];
+    const int c = threadIdx.x & 31, r = threadIdx.x >> 5;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (t0 + r + 8 * i < len) s[r + 8 * i][c] = x[(off + t0 + r + 8 * i) * D + d0 + c];
+    __syncthreads();
+    if (t0 + c >= len) return;
+#pragma unroll
+    for (int i = 0; i < 4; i++) out[off * D + (int64_t) (d0 + r + 8 * i) * len + t0 + c] = s[c][r + 8 * i];
+}
+
 float half_to_float(uint16_t h) {
     const uint32_t s = (uint32_t) (h >> 15) << 31;
     uint32_t e = (h >> 10) & 31, f = h & 1023, u;
@@ -978,15 +999,13 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
         }
         GSVK_TRY(bert_ln(m, x, prj, s2, pst, w.ff2_b, w.ln2, rows, x, x16_for(li + 1), xq_for(li + 1), xqd));
     }
-    // [rows][D] -> per sequence [D][len] (src/gsv_bert.cpp:220-228)
-    GSVK_HIP(hipMemcpyAsync(m->pin, x, (size_t) rows * D * 4, hipMemcpyDeviceToHost, st));
+    // [rows][D] -> per sequence [D][len], on the device (on the host the strided walk took longer
+    // than all kernels: 2,200 rows 6.5 ms)
+    hipLaunchKernelGGL(k_bert_features, dim3((unsigned) ((Tmax + 31) / 32), (unsigned) (D / 32), (unsigned) B), dim3(256),
+                       0, st, x, d_off, d_len, D, qkv);
+    GSVK_LAUNCH_CHECK();
+    GSVK_HIP(hipMemcpyAsync(m->pin, qkv, (size_t) rows * D * 4, hipMemcpyDeviceToHost, st));
     GSVK_HIP(hipStreamSynchronize(st));
-    const float * host = (const float *) m->pin;
-    for (int b = 0; b < B; b++) {
-        float * ob = out + (size_t) D * off[b];
-        const float * hb = host + (size_t) off[b] * D;
-        for (int d = 0; d < D; d++)
-            for (int t = 0; t < len[b]; t++) ob[(size_t) d * len[b] + t] = hb[(size_t) t * D + d];
-    }
+    memcpy(out, m->pin, (size_t) rows * D * 4);
     return GSVK_OK;
 }

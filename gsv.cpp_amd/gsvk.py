@@ -540,7 +540,7 @@ class Bert:
         for b, q in enumerate(seqs):
             ids[b, :len(q)] = q
         D = self.info["hidden"]
-        out = np.zeros(D * int(lens.sum()), np.float32)
+        out = np.empty(D * int(lens.sum()), np.float32)
         check(lib().gsvk_bert_encode(self.h, len(seqs), ids.ctypes.data, lens.ctypes.data, T, n_layers,
                                      out.ctypes.data), "bert_encode")
         res, off = [], 0
