@@ -9,16 +9,19 @@
 //   x   = LN2(x + W2 . gelu_erf(W1 . x + b1) + b2)
 // Output [hidden][T] row-major per sequence (src/gsv_bert.cpp:220-228).
 //
-// Design: rows of all sequences packed back to back (no padding rows). The projections are
-// k_bert_gemm below, on the matrix cores: F32 weights in fp32 (v_mfma_f32_32x32x2f32, ggml-cpu's
-// F32 x F32 product), F16 weights kept in fp16 with the activations rounded to fp16 and fp32 sums
-// (v_mfma_f32_32x32x16_f16; ggml-cpu converts the activations to the weights' F16 dot type),
-// Q8_0 weight files widened to fp32 at load. A workgroup computes a 64-row x 32-column tile over
-// a K slice, its 8 waves an eighth of the slice each, loading their operands straight into
-// registers (16 bytes per lane, the next group of steps in flight while one is multiplied);
-// the 8 partial tiles are summed through LDS in a fixed order. For few rows the K range is split
-// over workgroups too, into partial rows that the consumer (the LayerNorm) sums in order, so
-// every result is the same from run to run. The FFN1 GEMM applies bias + GELU itself.
+// Design: rows of all sequences packed back to back (no padding rows). The projections run on the
+// matrix cores with fp32 sums: F16 weights kept in fp16 with the activations rounded to fp16
+// (ggml-cpu converts the activations to the weights' F16 dot type), F32 weights in fp32 precision
+// (ggml-cpu's F32 x F32 product), Q8_0 weights on the int8 GEMM of the AR path. Over many rows
+// they are the LDS-tiled k_bert_gemm_lds of bert_gemm.h, which takes fp32 values as three bf16
+// planes. Over few rows (one sentence, where the weights' arrival sets the time) they are
+// k_bert_gemm below: a workgroup computes a 64- or 32-row x 32-column tile over a K slice, its 8
+// waves an eighth of the slice each, loading their operands straight into registers (16 bytes per
+// lane, the next group of steps in flight while one is multiplied), F32 weights with
+// v_mfma_f32_32x32x2f32; the 8 partial tiles are summed through LDS in a fixed order. Where the
+// tiles are few the K range is split over workgroups too, into partial rows that the consumer (the
+// LayerNorm) sums in order. Every result is the same from run to run. The FFN1 GEMM applies bias +
+// GELU itself.
 // LayerNorm over the partial rows is k_bert_ln; attention is k_bert_attn below: one workgroup per
 // 16 queries of one (sequence, head), four lanes per query (a quarter of the head dims each),
 // keys and values staged through LDS in tiles of 64 whose 4 chunks of 16 keys go to its 4 waves
@@ -30,6 +33,7 @@
 #include <string>
 #include <vector>
 
+#include "bert_gemm.h"
 #include "common.h"
 #include "gguf.h"
 #include "layer.h"
@@ -43,15 +47,6 @@ constexpr int BA_HD = 64;   // head dim of the kernels below (BERT-large: 1024 /
 constexpr int BA_KT = 64;   // keys per LDS tile
 constexpr int BA_CH = 16;   // keys per softmax chunk
 constexpr int BA_Q = 16;    // queries per workgroup (4 lanes per query in each of its 4 waves)
-
-// fp16 GEMM operands (F16 weights and the activations that meet them) are kept in the order the
-// matrix cores read them: per 32-row tile and step of 16 K values a 1 KB chunk in which lane
-// L = 32 g + i holds row i's values [8 g, 8 g + 8) of the step, so that a wave's operand load is
-// one contiguous 1 KB. Offset (in halves) of element (r, k) of an [R][K] matrix, K % 16 == 0;
-// rows are padded to a multiple of 64 (the rows of one workgroup).
-__host__ __device__ inline int64_t bt_off(int64_t r, int64_t k, int64_t K) {
-    return ((((r >> 5) * (K >> 4) + (k >> 4)) << 9) + (((((k >> 3) & 1) << 5) | (r & 31)) << 3)) + (k & 7);
-}
 
 // x[r] = word[id_r] + pos[t_r] + type0 (the sum order of src/gsv_bert.cpp:141-144); one
 // workgroup of 256 threads per row, 4 values per thread and pass.
@@ -87,7 +82,8 @@ __global__ void __launch_bounds__(256) k_bert_attn(const float * __restrict__ qk
                                                    const int32_t * __restrict__ seq_off,
                                                    const int32_t * __restrict__ seq_len, int D,
                                                    float scale_log2, float * __restrict__ out,
-                                                   _Float16 * __restrict__ out16) {
+                                                   uint16_t * __restrict__ out16,
+                                                   uint16_t * __restrict__ out3) {
     const int h = blockIdx.y, b = blockIdx.z;
     const int len = seq_len[b];
     const int64_t off = seq_off[b];
@@ -206,23 +202,22 @@ __global__ void __launch_bounds__(256) k_bert_attn(const float * __restrict__ qk
     }
     const float inv = 1.0f / L;
     const int64_t o0 = (off + q0 + qq) * (int64_t) D + h * BA_HD + 16 * c;
-    if (out16) {   // the fp16 input of an F16 out projection, in the operand order
+#pragma unroll
+    for (int i = 0; i < 16; i++) O[i] = O[i] * inv;
+    if (out16 || out3) {   // the input of an F16 / F32 out projection, in the operand order
         const int64_t row = off + q0 + qq;
         const int d0 = h * BA_HD + 16 * c;
 #pragma unroll
         for (int hh = 0; hh < 2; hh++) {
-            uint32_t w[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                w[j] = (uint32_t) f2h(O[8 * hh + 2 * j] * inv) | ((uint32_t) f2h(O[8 * hh + 2 * j + 1] * inv) << 16);
-            *reinterpret_cast<uint4 *>(out16 + bt_off(row, d0 + 8 * hh, D)) = make_uint4(w[0], w[1], w[2], w[3]);
+            if (out16) store_op16<8>(out16 + bt_off<1>(row, d0 + 8 * hh, D), O + 8 * hh);
+            if (out3) store_op3<8>(out3 + bt_off<3>(row, d0 + 8 * hh, D), O + 8 * hh);
         }
         return;
     }
     float4 * op = reinterpret_cast<float4 *>(out + o0);
 #pragma unroll
     for (int i = 0; i < 4; i++)
-        op[i] = make_float4(O[4 * i] * inv, O[4 * i + 1] * inv, O[4 * i + 2] * inv, O[4 * i + 3] * inv);
+        op[i] = make_float4(O[4 * i], O[4 * i + 1], O[4 * i + 2], O[4 * i + 3]);
 }
 
 // The features [rows][D] as the caller takes them, [D][len_b] per sequence, the sequences back to
@@ -270,8 +265,9 @@ float half_to_float(uint16_t h) {
 // A projection weight [N][K]: fp16 bits when the file holds F16 (multiplied as ggml-cpu does,
 // with the activations rounded to fp16 and fp32 accumulation), else fp32.
 struct Proj {
-    void * w = nullptr;
+    void * w = nullptr;         // F16: operand order (bt_off<1>); F32: fp32, row-major
     bool f16 = false;
+    uint16_t * w3 = nullptr;    // F32: the three bf16 planes too, in the operand order (bt_off<3>)
     // Q8_0 weights: natural-order quants [N][K] and fp16 scales [N][K/32], multiplied on the int8
     // GEMM with the activations quantised as ggml-cpu quantises them (its vec_dot type for Q8_0)
     int8_t * q8 = nullptr;
@@ -284,27 +280,13 @@ struct BertLayer {
     float * ff1_b = nullptr, * ff2_b = nullptr, * ln2 = nullptr;
 };
 
-typedef _Float16 bv8h __attribute__((ext_vector_type(8)));
-typedef float bv16f __attribute__((ext_vector_type(16)));
-
-constexpr int BG_BM = 64;        // most rows per workgroup (two 32-row MFMA tiles per wave)
 constexpr int BG_BN = 32;        // columns per workgroup
 constexpr int BG_WAVES = 8;      // each an eighth of the workgroup's K slice
 constexpr int BG_U = 4;          // MFMA steps per group of loads
 
-// Output stage of k_bert_gemm. With a K slice per workgroup (gridDim.z > 1) only y is written:
-// slice z of the sum to y + z * pstride (partial rows, summed by their consumer).
-struct BgOut {
-    float * y;            // [M][N] fp32, or null
-    int64_t pstride;      // floats between partial slices
-    const float * bias;   // added before the activation, or null
-    int gelu;             // y = gelu_erf(y + bias) (the add_act of src/gsv_bert.cpp:151-153)
-    _Float16 * y16;       // fp16 copy (nearest even) in the operand order (bt_off), or null
-};
-
 // K values of one MFMA step and of one 16-byte lane load, per operand type
 template <typename T> struct BgStep;
-template <> struct BgStep<_Float16> { static constexpr int K = 16, PER_LOAD = 8; };
+template <> struct BgStep<_Float16> { static constexpr int K = 16; };
 template <> struct BgStep<float> { static constexpr int K = 8, PER_LOAD = 4; };
 
 // Y[M][N] (or a K slice of it) = X[M][K] . W[N][K]^T, 8 waves each an eighth of the K slice (so
@@ -426,33 +408,30 @@ __global__ void __launch_bounds__(BG_WAVES * 64) k_bert_gemm(const T * __restric
     }
     if (o.gelu) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) y[j] = 0.5f * y[j] * (1.0f + erff(y[j] * 0.70710678118654752440f));
+        for (int j = 0; j < 8; j++) y[j] = bert_gelu(y[j]);
     }
     if (o.y) {
         float * yr = o.y + (int64_t) p * o.pstride + (int64_t) row * N + col;
         *reinterpret_cast<float4 *>(yr) = make_float4(y[0], y[1], y[2], y[3]);
         *reinterpret_cast<float4 *>(yr + 4) = make_float4(y[4], y[5], y[6], y[7]);
     }
-    if (o.y16) {   // in the operand order of the next GEMM (K = N)
-        uint32_t h[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) h[j] = (uint32_t) f2h(y[2 * j]) | ((uint32_t) f2h(y[2 * j + 1]) << 16);
-        *reinterpret_cast<uint4 *>(o.y16 + bt_off(row, col, N)) = make_uint4(h[0], h[1], h[2], h[3]);
-    }
+    if (o.y16) store_op16<8>(o.y16 + bt_off<1>(row, col, N), y);   // the next GEMM's operand (K = N)
+    if (o.y3) store_op3<8>(o.y3 + bt_off<3>(row, col, N), y);
 }
 
 // LayerNorm((x + (r_0 + r_1 + ... + r_{np-1})) + bias) * w + b of one row of n = 4 x 256 values
 // per workgroup (4 values per thread), r the np <= 8 partial rows of a split-K projection (np = 1:
 // the projection's output; r null: x alone), every load issued before the first use. The
 // LayerNorm of norm.hip otherwise: sums in double, var = E[v^2] - mean^2,
-// y = fma((v - mean) * inv, w, b); y16 its fp16 copy in the operand order (bt_off).
+// y = fma((v - mean) * inv, w, b); y16 / y3 its fp16 / three-plane copy in the operand order.
 constexpr int BL_THREADS = 256;
 constexpr int BL_MAXP = 8;
 __global__ void __launch_bounds__(BL_THREADS) k_bert_ln(const float * __restrict__ x, const float * __restrict__ r,
                                                         int np, int64_t pstride, const float * __restrict__ bias,
                                                         const float * __restrict__ wb, int n, float eps,
-                                                        float * __restrict__ y, _Float16 * __restrict__ y16,
-                                                        int8_t * __restrict__ yq, float * __restrict__ yd) {
+                                                        float * __restrict__ y, uint16_t * __restrict__ y16,
+                                                        uint16_t * __restrict__ y3, int8_t * __restrict__ yq,
+                                                        float * __restrict__ yd) {
     __shared__ double s_red[2][BL_THREADS / 64];
     const int64_t row = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -507,11 +486,8 @@ __global__ void __launch_bounds__(BL_THREADS) k_bert_ln(const float * __restrict
 #pragma unroll
     for (int i = 0; i < 4; i++) out[i] = __builtin_fmaf((v[i] - mean) * inv, wv4[i], cv4[i]);
     *reinterpret_cast<float4 *>(y + o) = make_float4(out[0], out[1], out[2], out[3]);
-    if (y16) {   // in the operand order of the next GEMM (K = n)
-        const uint32_t h0 = (uint32_t) f2h(out[0]) | ((uint32_t) f2h(out[1]) << 16);
-        const uint32_t h1 = (uint32_t) f2h(out[2]) | ((uint32_t) f2h(out[3]) << 16);
-        *reinterpret_cast<uint2 *>(y16 + bt_off(row, c, n)) = make_uint2(h0, h1);
-    }
+    if (y16) store_op16<4>(y16 + bt_off<1>(row, c, n), out);   // the next GEMM's operand (K = n)
+    if (y3) store_op3<4>(y3 + bt_off<3>(row, c, n), out);
     if (yq) {   // the x86 Q8_0 quantisation of the row (natural order): a block is 8 threads
         int8_t q[4];
         const float d = q8_quantize_group<4>(out, q, 8);
@@ -529,11 +505,22 @@ __global__ void __launch_bounds__(256) k_bert_gelu_q8(const float * __restrict__
     const float4 v = *reinterpret_cast<const float4 *>(h + i);
     float y[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int k = 0; k < 4; k++) y[k] = 0.5f * y[k] * (1.0f + erff(y[k] * 0.70710678118654752440f));
+    for (int k = 0; k < 4; k++) y[k] = bert_gelu(y[k]);
     int8_t q[4];
     const float d = q8_quantize_group<4>(y, q, 8);
     *reinterpret_cast<int *>(hq + i) = (q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((q[3] & 0xff) << 24);
     if ((i & 31) == 0) hd[i / 32] = d;
+}
+
+// An fp32 matrix [R][K] (R % 32 == 0, K % 16 == 0) as three bf16 planes in the operand order: 8
+// values per thread.
+__global__ void __launch_bounds__(256) k_bert_planes(const float * __restrict__ w, int64_t n, int64_t K,
+                                                     uint16_t * __restrict__ w3) {
+    const int64_t i = ((int64_t) blockIdx.x * 256 + threadIdx.x) * 8;
+    if (i >= n) return;
+    const float4 a = *reinterpret_cast<const float4 *>(w + i), b = *reinterpret_cast<const float4 *>(w + i + 4);
+    const float y[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    store_op3<8>(w3 + bt_off<3>(i / K, i % K, K), y);
 }
 
 }  // namespace
@@ -547,6 +534,7 @@ struct gsvk_bert {
     gsvk_bert_info info{};
     std::vector<void *> wmem;   // weight allocations
     bool any_f16 = false;       // some projection is kept in fp16
+    bool any_f32 = false;       // some projection is kept in fp32 (and as planes)
     bool any_q8 = false;        // some projection is Q8_0 (int8 GEMM)
     float * word = nullptr, * pos = nullptr, * type0 = nullptr, * emb_ln = nullptr;
     std::vector<BertLayer> L;
@@ -627,7 +615,7 @@ int load_tensor(gsvk_bert * m, const GgufFile & g, const std::string & name, int
         std::vector<uint16_t> tiled(n);
         const uint16_t * src = (const uint16_t *) raw.data();
         for (int64_t r = 0; r < ne1; r++)
-            for (int64_t k = 0; k < ne0; k++) tiled[bt_off(r, k, ne0)] = src[r * ne0 + k];
+            for (int64_t k = 0; k < ne0; k++) tiled[bt_off<1>(r, k, ne0)] = src[r * ne0 + k];
         uint16_t * w16 = nullptr;
         GSVK_TRY(m->dev_alloc(w16, n));
         GSVK_HIP(hipMemcpy(w16, tiled.data(), n * 2, hipMemcpyHostToDevice));
@@ -674,6 +662,13 @@ int load_tensor(gsvk_bert * m, const GgufFile & g, const std::string & name, int
     if (proj) {
         proj->w = out;
         proj->f16 = false;
+        GSVK_REQUIRE(ne0 % 16 == 0 && ne1 % 32 == 0, "BERT GGUF: %s: projection shape [%lld, %lld] (K %% 16, N %% 32)",
+                     name.c_str(), (long long) ne0, (long long) ne1);
+        GSVK_TRY(m->dev_alloc(proj->w3, 3 * n));
+        hipLaunchKernelGGL(k_bert_planes, dim3((unsigned) ((n / 8 + 255) / 256)), dim3(256), 0, m->stream, out, (int64_t) n,
+                           ne0, proj->w3);
+        GSVK_LAUNCH_CHECK();
+        m->any_f32 = true;
     }
     return GSVK_OK;
 }
@@ -695,14 +690,58 @@ int load_ln(gsvk_bert * m, const GgufFile & g, const std::string & wn, const std
     return GSVK_OK;
 }
 
+// Rows above which the LDS-tiled GEMM takes the projections; at most these the direct loads, which
+// put every weight's load in flight at once. Whole encode of one sequence, us, direct / tiled:
+//   F16  64 rows 825 / 1316, 256 rows 1403 / 1750, 384 rows 1870 / 2060, 512 rows 2105 / 2215;
+//        2265 rows (16 sequences) 5330 / 4845
+//   F32  64 rows 1257 / 1702, 96 rows 1836 / 1792, 128 rows 1855 / 1834, 160 rows 2845 / 2055,
+//        512 rows 5103 / 3425
+// (the F16 lines meet near 600 rows, the F32 lines near 90; the step at 128 -> 160 is a third row tile)
+constexpr int64_t BERT_DIRECT_ROWS_F16 = 512;
+constexpr int64_t BERT_DIRECT_ROWS_F32 = 96;
+bool bert_lds(const Proj & w, int64_t M) { return M > (w.f16 ? BERT_DIRECT_ROWS_F16 : BERT_DIRECT_ROWS_F32); }
+
+// The LDS-tiled GEMM's shapes: rows and columns per workgroup, steps per stage. F16: 128 x 128 where
+// that still gives a workgroup per CU, else 64 x 128 (2265 rows: FFN1 32.4 against 37.7 us, out and
+// FFN2, where it would leave 144 workgroups, 40.9 against 36.0). F32 (six products per step): 64 x 64
+// (564 rows, FFN1 33.6 us, 128 x 64 37.4, 128 x 128 38.8; the fp32 matrix instruction took 79).
+struct BgTile { int bm, bn, ks; };
+BgTile bert_tile(bool f16, int64_t M, int N) {
+    if (!f16) return {64, 64, 1};
+    return {((M + 127) / 128) * (N / 128) >= 256 ? 128 : 64, 128, 4};
+}
+
+template <int PL, int TM, int TN, int WM, int WN, int KS, int NBUF>
+int launch_bert_lds(gsvk_bert * m, const uint16_t * X, const uint16_t * W, int64_t M, int N, int K, int slices,
+                    const BgOut & o) {
+    constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
+    const int64_t tiles = (M + BM - 1) / BM * (N / BN) * slices;
+    GSVK_REQUIRE(N % BN == 0 && K % (16 * KS * slices) == 0 && tiles < (1ll << 31) && BG_ROW_PAD % BM == 0,
+                 "bert gemm: unsupported shape M=%lld N=%d K=%d slices %d", (long long) M, N, K, slices);
+    // an XCD's run of tiles reads the smaller operand whole, so the larger one is split over the XCDs
+    hipLaunchKernelGGL((k_bert_gemm_lds<PL, TM, TN, WM, WN, KS, NBUF>), dim3((unsigned) tiles), dim3(64 * WM * WN), 0,
+                       m->stream, X, W, (int) M, N, K, slices, (int) (M < N), o);
+    GSVK_LAUNCH_CHECK();
+    return GSVK_OK;
+}
+
 // Row tiles of 32 per wave: 2 (64-row workgroups) when that still gives 256 workgroups, else 1.
 int bert_row_tiles(int64_t M, int N) {
     return M > 32 && (int64_t) (N / BG_BN) * ((M + 63) / 64) >= 256 ? 2 : 1;
 }
 
-// K slices for an [M][N][K] projection: enough workgroups (row x 32-column tiles x slices) to
-// cover the chip when the rows are few, each slice a multiple of the kernel's waves x steps.
-int bert_kslices(int64_t M, int N, int K, int kmult, int max_slices) {
+// K slices for an [M][N][K] projection: enough workgroups (tiles x slices) to cover the chip when the
+// tiles are few, each slice a multiple of what the kernel takes at a time. Tiled F32: two workgroups
+// per CU (564 rows, FFN2: 4 slices 33 us, 8 slices 31.5, which the LayerNorm's reads give back).
+int bert_kslices(const Proj & w, int64_t M, int N, int K, int max_slices) {
+    if (bert_lds(w, M)) {
+        const BgTile t = bert_tile(w.f16, M, N);
+        const int64_t tiles = (M + t.bm - 1) / t.bm * (N / t.bn);
+        int p = 1;
+        while (p < max_slices && tiles * p < (w.f16 ? 256 : 512) && K % (2 * p * 16 * t.ks) == 0) p *= 2;
+        return p;
+    }
+    const int kmult = BG_WAVES * BG_U * (w.f16 ? BgStep<_Float16>::K : BgStep<float>::K);
     const int bm = 32 * bert_row_tiles(M, N);
     const int64_t tiles = (int64_t) (N / BG_BN) * ((M + bm - 1) / bm);
     int p = 1;
@@ -710,14 +749,27 @@ int bert_kslices(int64_t M, int N, int K, int kmult, int max_slices) {
     return p;
 }
 
-// Y = X . W^T for W of the projection's type (fp16 operands when W is F16: X16 holds the
-// activations already rounded by their producer; fp32 otherwise); `slices` K slices (> 1: partial
+// Y = X . W^T for W of the projection's type (W F16: X16 holds the activations already rounded by
+// their producer; W F32: X, or over many rows their planes X3); `slices` K slices (> 1: partial
 // rows at Y + z * M * N, bias / GELU / y16 not allowed).
-int gemm(gsvk_bert * m, const Proj & W, const float * X, const _Float16 * X16, int64_t M, int N, int K,
-         int slices, const BgOut & o) {
+int gemm(gsvk_bert * m, const Proj & W, const float * X, const uint16_t * X16, const uint16_t * X3, int64_t M, int N,
+         int K, int slices, const BgOut & o) {
     const int kmult = BG_WAVES * BG_U * (W.f16 ? BgStep<_Float16>::K : BgStep<float>::K);
-    GSVK_REQUIRE(M > 0 && M < (1 << 30) && N % BG_BN == 0 && slices >= 1 && K % (slices * kmult) == 0 &&
-                     (slices == 1 || (!o.bias && !o.gelu && !o.y16)) && (o.y || o.y16),
+    GSVK_REQUIRE(M > 0 && M < (1 << 30) && slices >= 1 &&
+                     (slices == 1 || (!o.bias && !o.gelu && !o.y16 && !o.y3)) && (o.y || o.y16 || o.y3),
+                 "bert gemm: unsupported shape M=%lld N=%d K=%d slices %d", (long long) M, N, K, slices);
+    if (bert_lds(W, M)) {
+        if (!W.f16) {
+            GSVK_REQUIRE(X3 && W.w3, "bert gemm: F32 weights over many rows need the planes");
+            return launch_bert_lds<3, 1, 1, 2, 2, 1, 4>(m, X3, W.w3, M, N, K, slices, o);
+        }
+        GSVK_REQUIRE(X16, "bert gemm: F16 weights need fp16 activations");
+        const uint16_t * w16 = (const uint16_t *) W.w;
+        if (bert_tile(true, M, N).bm == 128)
+            return launch_bert_lds<1, 2, 2, 2, 2, 2, 3>(m, X16, w16, M, N, K, slices, o);
+        return launch_bert_lds<1, 1, 2, 2, 2, 4, 3>(m, X16, w16, M, N, K, slices, o);
+    }
+    GSVK_REQUIRE(N % BG_BN == 0 && K % (slices * kmult) == 0,
                  "bert gemm: unsupported shape M=%lld N=%d K=%d slices %d", (long long) M, N, K, slices);
     const int rt = bert_row_tiles(M, N);
     const dim3 grid((unsigned) (N / BG_BN), (unsigned) ((M + 32 * rt - 1) / (32 * rt)), (unsigned) slices);
@@ -743,7 +795,7 @@ int gemm(gsvk_bert * m, const Proj & W, const float * X, const _Float16 * X16, i
     }
     if (W.f16) {
         GSVK_REQUIRE(X16, "bert gemm: F16 weights need fp16 activations");
-        GSVK_BG_ALL(_Float16, X16, (const _Float16 *) W.w);
+        GSVK_BG_ALL(_Float16, (const _Float16 *) X16, (const _Float16 *) W.w);
     } else {
         GSVK_REQUIRE(X, "bert gemm: F32 weights need fp32 activations");
         GSVK_BG_ALL(float, X, (const float *) W.w);
@@ -770,13 +822,13 @@ int gemm_q8(gsvk_bert * m, const Proj & W, const int8_t * xq, const float * xd, 
 }
 
 int bert_ln(gsvk_bert * m, const float * x, const float * r, int np, int64_t pstride, const float * bias,
-            const float * wb, int64_t rows, float * y, _Float16 * y16, int8_t * yq = nullptr,
+            const float * wb, int64_t rows, float * y, uint16_t * y16, uint16_t * y3, int8_t * yq = nullptr,
             float * yd = nullptr) {
     const int D = m->info.hidden;
     GSVK_REQUIRE(D % 4 == 0 && D <= 4 * BL_THREADS && np >= 1 && np <= BL_MAXP,
                  "bert layernorm: hidden %d (<= %d), %d partial rows", D, 4 * BL_THREADS, np);
     hipLaunchKernelGGL(k_bert_ln, dim3((unsigned) rows), dim3(BL_THREADS), 0, m->stream, x, r, np, pstride, bias,
-                       wb, D, m->info.ln_eps, y, y16, yq, yd);
+                       wb, D, m->info.ln_eps, y, y16, y3, yq, yd);
     GSVK_LAUNCH_CHECK();
     return GSVK_OK;
 }
@@ -899,10 +951,11 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
     // rows), FFN hidden, the fp16 GEMM inputs (a D-wide row, the FFN hidden), the small arrays
     constexpr int BERT_MAX_SLICES = 8;
     const size_t fl = (size_t) rows * (D + 3 * D + D + (size_t) BERT_MAX_SLICES * D + F);
-    const int64_t rows64 = (rows + BG_BM - 1) / BG_BM * BG_BM;   // fp16 operands: rows padded to 64
-    const size_t n16 = m->any_f16 ? (size_t) rows64 * (D + F) : 0;
+    const int64_t rowsp = (rows + BG_ROW_PAD - 1) / BG_ROW_PAD * BG_ROW_PAD;   // rows of the operand order
+    const size_t n16 = m->any_f16 ? (size_t) rowsp * (D + F) : 0;
+    const size_t n3 = m->any_f32 && rows > BERT_DIRECT_ROWS_F32 ? (size_t) rowsp * (D + F) * 3 : 0;
     const size_t nq = m->any_q8 ? (size_t) rows * (D + F) : 0;   // Q8_0 activations: quants
-    const size_t need = fl * 4 + n16 * 2 + nq + (nq / 32) * 4 + (size_t) rows * 8 + (size_t) B * 8 + 8192;
+    const size_t need = fl * 4 + (n16 + n3) * 2 + nq + (nq / 32) * 4 + (size_t) rows * 8 + (size_t) B * 8 + 8192;
     if (need > m->ws_bytes) {
         if (m->ws) (void) hipFree(m->ws);
         m->ws = nullptr;
@@ -920,9 +973,11 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
     float * att = qkv + rows * 3 * D;
     float * prj = att + rows * D;
     float * h = prj + (size_t) BERT_MAX_SLICES * rows * D;
-    _Float16 * x16 = (_Float16 *) (h + rows * F);            // fp16 input of the D-wide projections
-    _Float16 * h16 = m->any_f16 ? x16 + rows64 * D : nullptr;   // fp16 FFN hidden (FFN2's input)
-    int8_t * xq = (int8_t *) (x16 + n16);                          // D-wide Q8_0 rows (+ scales)
+    uint16_t * x16 = (uint16_t *) (h + rows * F);            // fp16 input of the D-wide projections
+    uint16_t * h16 = m->any_f16 ? x16 + rowsp * D : nullptr;    // fp16 FFN hidden (FFN2's input)
+    uint16_t * x3 = x16 + n16;                                  // the same as planes, for F32 projections
+    uint16_t * h3 = x3 + (n3 ? rowsp * D * 3 : 0);
+    int8_t * xq = (int8_t *) (x3 + n3);                          // D-wide Q8_0 rows (+ scales)
     int8_t * hq = xq + (m->any_q8 ? rows * D : 0);                  // the FFN hidden's
     float * xqd = (float *) (((uintptr_t) (xq + nq) + 15) & ~(uintptr_t) 15);
     float * hqd = xqd + (m->any_q8 ? rows * D / 32 : 0);
@@ -952,13 +1007,14 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
     hipLaunchKernelGGL(k_bert_embed, dim3((unsigned) rows), dim3(256), 0, st, m->word, m->pos, m->type0, d_ids,
                        d_pos, D, prj);
     GSVK_LAUNCH_CHECK();
-    // each LayerNorm also writes the fp16 copy (F16 consumer) or the Q8_0 rows (Q8_0 consumer) its
-    // consumer takes
+    // each LayerNorm also writes the fp16 copy (F16 consumer), the planes (F32 consumer, many rows) or
+    // the Q8_0 rows (Q8_0 consumer) its consumer takes
+    auto w3 = [&](const Proj & w) { return w.w3 && bert_lds(w, rows); };
     auto x16_for = [&](int li) { return li < n_layers && m->L[li].qkv.f16 ? x16 : nullptr; };
+    auto x3_for = [&](int li) { return li < n_layers && w3(m->L[li].qkv) ? x3 : nullptr; };
     auto xq_for = [&](int li) { return li < n_layers && m->L[li].qkv.q8 ? xq : nullptr; };
-    GSVK_TRY(bert_ln(m, prj, nullptr, 1, 0, nullptr, m->emb_ln, rows, x, x16_for(0), xq_for(0), xqd));
+    GSVK_TRY(bert_ln(m, prj, nullptr, 1, 0, nullptr, m->emb_ln, rows, x, x16_for(0), x3_for(0), xq_for(0), xqd));
     const float scale_log2 = 1.4426950408889634f / std::sqrt((float) BA_HD);
-    auto kmult = [](const Proj & w) { return BG_WAVES * BG_U * (w.f16 ? BgStep<_Float16>::K : BgStep<float>::K); };
     const int64_t pst = rows * D;   // floats between partial rows of the D-wide projections
     for (int li = 0; li < n_layers; li++) {
         const BertLayer & w = m->L[li];
@@ -966,10 +1022,10 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
         if (w.qkv.q8)
             GSVK_TRY(gemm_q8(m, w.qkv, xq, xqd, rows, 3 * D, D, qkv, nullptr));
         else
-            GSVK_TRY(gemm(m, w.qkv, x, x16, rows, 3 * D, D, 1, BgOut{qkv, 0, nullptr, 0, nullptr}));
+            GSVK_TRY(gemm(m, w.qkv, x, x16, x3, rows, 3 * D, D, 1, BgOut{qkv, 0, nullptr, 0, nullptr, nullptr}));
         hipLaunchKernelGGL(k_bert_attn, dim3((unsigned) ((Tmax + BA_Q - 1) / BA_Q), (unsigned) in.heads, (unsigned) B),
                            dim3(256), 0, st, qkv, w.qkv_b, d_off, d_len, D, scale_log2, att,
-                           w.ao.f16 ? x16 : nullptr);
+                           w.ao.f16 ? x16 : nullptr, w3(w.ao) ? x3 : nullptr);
         GSVK_LAUNCH_CHECK();
         // out projection (F16 / F32: in K slices when the rows are few; LN1 sums the slices)
         int s1 = 1;
@@ -977,11 +1033,11 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
             GSVK_TRY(launch_q8_quantize(att, rows, D, xq, xqd, st, Q8_NATURAL));
             GSVK_TRY(gemm_q8(m, w.ao, xq, xqd, rows, D, D, prj, nullptr));
         } else {
-            s1 = bert_kslices(rows, D, D, kmult(w.ao), BERT_MAX_SLICES);
-            GSVK_TRY(gemm(m, w.ao, att, x16, rows, D, D, s1, BgOut{prj, pst, nullptr, 0, nullptr}));
+            s1 = bert_kslices(w.ao, rows, D, D, BERT_MAX_SLICES);
+            GSVK_TRY(gemm(m, w.ao, att, x16, x3, rows, D, D, s1, BgOut{prj, pst, nullptr, 0, nullptr, nullptr}));
         }
         GSVK_TRY(bert_ln(m, x, prj, s1, pst, w.ao_b, w.ln1, rows, x, w.ff1.f16 ? x16 : nullptr,
-                         w.ff1.q8 ? xq : nullptr, xqd));
+                         w3(w.ff1) ? x3 : nullptr, w.ff1.q8 ? xq : nullptr, xqd));
         // FFN1 + bias + GELU, FFN2
         int s2 = 1;
         if (w.ff1.q8) {
@@ -991,13 +1047,16 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
             GSVK_LAUNCH_CHECK();
             GSVK_TRY(gemm_q8(m, w.ff2, hq, hqd, rows, D, F, prj, nullptr));
         } else {
-            // bias + GELU in the FFN1 epilogue, to fp32 (an F32 FFN2) or fp16 (an F16 FFN2)
-            GSVK_TRY(gemm(m, w.ff1, x, x16, rows, F, D, 1,
-                          BgOut{w.ff2.f16 ? nullptr : h, 0, w.ff1_b, 1, w.ff2.f16 ? h16 : nullptr}));
-            s2 = bert_kslices(rows, D, F, kmult(w.ff2), BERT_MAX_SLICES);
-            GSVK_TRY(gemm(m, w.ff2, h, h16, rows, D, F, s2, BgOut{prj, pst, nullptr, 0, nullptr}));
+            // bias + GELU in the FFN1 epilogue, to fp16 (an F16 FFN2), planes or fp32 (an F32 FFN2)
+            const bool f2w3 = w3(w.ff2);
+            GSVK_TRY(gemm(m, w.ff1, x, x16, x3, rows, F, D, 1,
+                          BgOut{w.ff2.f16 || f2w3 ? nullptr : h, 0, w.ff1_b, 1, w.ff2.f16 ? h16 : nullptr,
+                                f2w3 ? h3 : nullptr}));
+            s2 = bert_kslices(w.ff2, rows, D, F, BERT_MAX_SLICES);
+            GSVK_TRY(gemm(m, w.ff2, h, h16, h3, rows, D, F, s2, BgOut{prj, pst, nullptr, 0, nullptr, nullptr}));
         }
-        GSVK_TRY(bert_ln(m, x, prj, s2, pst, w.ff2_b, w.ln2, rows, x, x16_for(li + 1), xq_for(li + 1), xqd));
+        GSVK_TRY(bert_ln(m, x, prj, s2, pst, w.ff2_b, w.ln2, rows, x, x16_for(li + 1), x3_for(li + 1),
+                         xq_for(li + 1), xqd));
     }
     // [rows][D] -> per sequence [D][len], on the device (on the host the strided walk took longer
     // than all kernels: 2,200 rows 6.5 ms)

@@ -105,6 +105,27 @@ def test_quantised_weight_files(gpu, tmp_path_factory, wtype, T):
         m.close()
 
 
+@pytest.mark.parametrize("wtype,lens", [
+    ("f32", (96,)), ("f32", (97,)), ("f32", (64, 1, 64)), ("f32", (300, 3, 210)),   # direct / planes, tiles + 1
+    ("f16", (512,)), ("f16", (512, 1)), ("f16", (400, 240, 1)),                     # direct / 64-row tiles
+    ("f16", (512, 512, 1)), ("f16", (301, 512, 150, 62)),                            # 128-row tiles: 1025 rows
+])
+def test_tiled_projections(gpu, tmp_path_factory, wtype, lens):
+    """The LDS-tiled GEMM at the edges of its tiles and of its dispatch. F32 rows (three bf16 planes)
+    also within fp32 rounding: 2e-6 of the scale (measured 3e-7; a product of plain bf16 planes h + m
+    would be 2^-17 = 8e-6 off)."""
+    m, W = _model(tmp_path_factory, wtype, 2, 1)
+    try:
+        rng = np.random.default_rng(sum(lens))
+        seqs = [_ids(rng, n) for n in lens]
+        for q, got in zip(seqs, m.encode(seqs)):
+            err = _check(got, BO.encode(W, q, 1, 1024, 16, 1e-12, act_f16=wtype == "f16"))
+            if wtype == "f32":
+                assert err <= 2e-6, err
+    finally:
+        m.close()
+
+
 def test_gsv_bert_class_drop_in(bert_f32, tmp_path_factory):
     """The C++ gsv_bert class (include/gsv_bert.h) through every member, driven by
     tests/dropin/gsv_bert_check.cpp (built by oracle/Makefile, target bertcheck)."""
