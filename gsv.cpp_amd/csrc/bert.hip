@@ -22,7 +22,8 @@
 // tiles are few the K range is split over workgroups too, into partial rows that the consumer (the
 // LayerNorm) sums in order. Every result is the same from run to run. The FFN1 GEMM applies bias +
 // GELU itself.
-// LayerNorm over the partial rows is k_bert_ln; attention is k_bert_attn below: one workgroup per
+// LayerNorm over the partial rows is k_bert_ln. Attention is k_bert_attn_mfma on the matrix cores, or
+// where that gives few workgroups k_bert_attn, both below. The latter takes one workgroup per
 // 16 queries of one (sequence, head), four lanes per query (a quarter of the head dims each),
 // keys and values staged through LDS in tiles of 64 whose 4 chunks of 16 keys go to its 4 waves
 // (online softmax each, merged at the end), fp32 throughout.
@@ -218,6 +219,187 @@ __global__ void __launch_bounds__(256) k_bert_attn(const float * __restrict__ qk
 #pragma unroll
     for (int i = 0; i < 4; i++)
         op[i] = make_float4(O[4 * i], O[4 * i + 1], O[4 * i + 2], O[4 * i + 3]);
+}
+
+// The same attention on the matrix cores, for longer sequences, every product as the six bf16
+// products of three planes (bert_gemm.h), fp32 sums. Workgroup = 4 waves x 32 queries of one
+// (sequence, head); key tiles of 32 staged through LDS as planes in the operand order, double
+// buffered (the next tile is fetched into registers before this one is used).
+//   scores, transposed: S^T[key][query] = K . Q^T, so a lane holds 16 keys of query lane % 32 and the
+//     online softmax is in-lane plus one exchange with lane ^ 32;
+//   output, transposed: O^T[dim][query] += V^T . P^T, with P^T straight from the score registers:
+//     K slot (c, g) of the product holds the keys 16 c + 4 g + [0, 4) and 16 c + 8 + 4 g + [0, 4), and
+//     V^T is staged in that order. A tile's sum starts at zero (its small products first) and joins
+//     the running one in one fma with the rescaling.
+// It is bound by its instructions per tile (splits and softmax on the vector ALUs beside 48 products):
+// 16 sequences of 5 to 301 tokens 64.4 -> 33.2 us per layer, 8 of 33 to 97 16.7 -> 15.8.
+// LDS: K chunk (step s of 16 dims, plane): slot 32 g + (key ^ (2 s + g)), so that the 8 threads that
+// write a key's 8 dim groups hit different banks; V^T chunk (dim tile, c, plane): slot 32 g + dim % 32.
+constexpr int BM_Q = 128;   // queries per workgroup
+struct BmTile {
+    uint4 k[4][3][64];
+    uint4 v[2][2][3][64];
+};
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_bert_attn_mfma(
+    const float * __restrict__ qkv, const float * __restrict__ qkv_b, const int32_t * __restrict__ seq_off,
+    const int32_t * __restrict__ seq_len, int D, float scale_log2, float * __restrict__ out,
+    uint16_t * __restrict__ out16, uint16_t * __restrict__ out3) {
+    const int h = blockIdx.y, b = blockIdx.z;
+    const int len = seq_len[b];
+    const int64_t off = seq_off[b];
+    if ((int) blockIdx.x * BM_Q >= len) return;   // uniform over the workgroup
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int li = lane & 31, lg = lane >> 5;
+    const int q0w = blockIdx.x * BM_Q + 32 * wave, q = q0w + li;
+    const int64_t rs = 3 * (int64_t) D;
+    const float * base = qkv + off * rs + h * BA_HD;
+    __shared__ BmTile tiles[2];
+
+    // staging: K, 8 dims of one key per thread; V, one dim of the 8 keys of a K slot
+    const int kkey = tid >> 3, kdg = tid & 7, vd = tid & 63, vc = tid >> 7, vg = (tid >> 6) & 1;
+    float kb[8];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float4 t = *reinterpret_cast<const float4 *>(qkv_b + D + h * BA_HD + 8 * kdg + 4 * i);
+        kb[4 * i] = t.x; kb[4 * i + 1] = t.y; kb[4 * i + 2] = t.z; kb[4 * i + 3] = t.w;
+    }
+    const float vb = qkv_b[2 * D + h * BA_HD + vd];
+    float4 fk[2];
+    float fv[8];
+    auto fetch = [&](int k0) {   // keys past the end repeat the last (masked below)
+        const float * kr = base + (int64_t) min(k0 + kkey, len - 1) * rs + D + 8 * kdg;
+        fk[0] = *reinterpret_cast<const float4 *>(kr);
+        fk[1] = *reinterpret_cast<const float4 *>(kr + 4);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            fv[i] = base[(int64_t) min(k0 + 16 * vc + 8 * (i >> 2) + 4 * vg + (i & 3), len - 1) * rs + 2 * D + vd];
+    };
+    // (a query, key or value beyond 2^127 would give NaN scores or outputs either way: its square
+    // overflows, and the LayerNorm after the attention turns an infinity into NaN)
+    auto planes = [&](const float * x, uint4 (&w)[3]) {
+        uint32_t s[3][4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) split3_pair(x[2 * i], x[2 * i + 1], s[0][i], s[1][i], s[2][i]);
+#pragma unroll
+        for (int p = 0; p < 3; p++) w[p] = make_uint4(s[p][0], s[p][1], s[p][2], s[p][3]);
+    };
+    auto store = [&](BmTile & t) {
+        const float x[8] = {fk[0].x + kb[0], fk[0].y + kb[1], fk[0].z + kb[2], fk[0].w + kb[3],
+                            fk[1].x + kb[4], fk[1].y + kb[5], fk[1].z + kb[6], fk[1].w + kb[7]};
+        uint4 w[3];
+        planes(x, w);
+#pragma unroll
+        for (int p = 0; p < 3; p++) t.k[kdg >> 1][p][32 * (kdg & 1) + (kkey ^ kdg)] = w[p];
+        float y[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) y[i] = fv[i] + vb;
+        planes(y, w);
+#pragma unroll
+        for (int p = 0; p < 3; p++) t.v[vd >> 5][vc][p][32 * vg + (vd & 31)] = w[p];
+    };
+
+    fetch(0);
+    uint4 qp[4][3];   // Q^T operand: query q, dims 16 s + 8 lg + [0, 8)
+    {
+        const float * qr = base + (int64_t) min(q, len - 1) * rs + 8 * lg;
+        const float * qb = qkv_b + h * BA_HD + 8 * lg;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            float x[8];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const float4 a = *reinterpret_cast<const float4 *>(qr + 16 * s + 4 * i);
+                const float4 c = *reinterpret_cast<const float4 *>(qb + 16 * s + 4 * i);
+                x[4 * i] = a.x + c.x; x[4 * i + 1] = a.y + c.y; x[4 * i + 2] = a.z + c.z; x[4 * i + 3] = a.w + c.w;
+            }
+            planes(x, qp[s]);
+        }
+    }
+    store(tiles[0]);
+    __syncthreads();
+
+    bv16f o[2] = {bv16f{}, bv16f{}};   // O^T: query q, dims 32 t + 8 (v / 4) + 4 lg + v % 4
+    float m = -INFINITY, l = 0.0f;
+    int buf = 0;
+    for (int k0 = 0; k0 < len; k0 += 32, buf ^= 1) {
+        const bool more = k0 + 32 < len;   // uniform
+        if (more) fetch(k0 + 32);
+        if (q0w < len) {                   // uniform per wave
+            const BmTile & t = tiles[buf];
+            bv16f sc = {}, sc1 = {};   // (two chains of dependent products)
+            uint4 a[4][3];
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int p = 0; p < 3; p++) a[s][p] = t.k[s][p][32 * lg + (li ^ (2 * s + lg))];
+#pragma unroll
+            for (int e = 0; e < 6; e++)
+#pragma unroll
+                for (int s = 0; s < 4; s += 2) {
+                    sc = mfma3(e, a[s], qp[s], sc);
+                    sc1 = mfma3(e, a[s + 1], qp[s + 1], sc1);
+                }
+#pragma unroll
+            for (int v = 0; v < 16; v++) sc[v] = sc[v] + sc1[v];
+            if (!more) {                   // the last tile may hold keys past the end
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    if (k0 + 8 * (v >> 2) + 4 * lg + (v & 3) >= len) sc[v] = -INFINITY;
+            }
+            float rmax = sc[0];
+#pragma unroll
+            for (int v = 1; v < 16; v++) rmax = fmaxf(rmax, sc[v]);
+            rmax = fmaxf(rmax, __shfl_xor(rmax, 32, 64));
+            const float mn = fmaxf(m, rmax * scale_log2);     // finite: the tile has a key
+            const float f = __builtin_amdgcn_exp2f(m - mn);   // 0 on the first tile (m = -inf)
+            float p[16], psum = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[v], scale_log2, -mn));
+                psum += p[v];
+            }
+            psum += __shfl_xor(psum, 32, 64);
+            l = __builtin_fmaf(l, f, psum);
+            m = mn;
+            uint4 pp[2][3];
+#pragma unroll
+            for (int c = 0; c < 2; c++) planes(p + 8 * c, pp[c]);
+            bv16f s[2] = {bv16f{}, bv16f{}};
+            uint4 x[2][2][3];
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int e = 0; e < 3; e++) x[dt][c][e] = t.v[dt][c][e][lane];
+#pragma unroll
+            for (int e = 0; e < 6; e++)
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int dt = 0; dt < 2; dt++) s[dt] = mfma3(e, x[dt][c], pp[c], s[dt]);
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) o[dt][v] = __builtin_fmaf(o[dt][v], f, s[dt][v]);
+        }
+        if (more) store(tiles[buf ^ 1]);
+        __syncthreads();
+    }
+    if (q >= len) return;
+    const float inv = 1.0f / l;
+    const int64_t row = off + q;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int col = h * BA_HD + 32 * dt + 8 * g + 4 * lg;
+            const float y[4] = {o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv};
+            if (out16) store_op16<4>(out16 + bt_off<1>(row, col, D), y);
+            if (out3) store_op3<4>(out3 + bt_off<3>(row, col, D), y);
+            if (!out16 && !out3) *reinterpret_cast<float4 *>(out + row * D + col) = make_float4(y[0], y[1], y[2], y[3]);
+        }
 }
 
 // The features [rows][D] as the caller takes them, [D][len_b] per sequence, the sequences back to
@@ -725,6 +907,13 @@ int launch_bert_lds(gsvk_bert * m, const uint16_t * X, const uint16_t * W, int64
     return GSVK_OK;
 }
 
+// Workgroups of the matrix-core attention (128 queries of a sequence and head each) above which it is
+// taken: with fewer the lane-per-query kernel's 8 times as many workgroups fill the chip better. Whole
+// encode of an F16 file, us, lane per query / matrix cores: 1 x 256 tokens (32 workgroups) 1406 / 1465,
+// 1 x 512, 2 x 256 and 4 x 64 (64) 2131 / 2142, 1817 / 1822 and 1215 / 1217, 8 x 32 and 8 x 64 (128)
+// 1203 / 1166 and 1617 / 1571, 16 x 200 (512) 6564 / 5104.
+constexpr int BERT_ATTN_WGS = 64;
+
 // Row tiles of 32 per wave: 2 (64-row workgroups) when that still gives 256 workgroups, else 1.
 int bert_row_tiles(int64_t M, int N) {
     return M > 32 && (int64_t) (N / BG_BN) * ((M + 63) / 64) >= 256 ? 2 : 1;
@@ -930,6 +1119,8 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
     if (n_layers < 0 || n_layers > in.layers_used) n_layers = in.layers_used;
     std::vector<int32_t> ids, tpos, off(B), len(B);
     int64_t rows = 0;
+    int Lmax = 0;   // the longest sequence (Tmax is the stride of ids_flat)
+    int64_t attn_wgs = 0;
     for (int b = 0; b < B; b++) {
         GSVK_REQUIRE(lens[b] >= 1 && lens[b] <= Tmax, "gsvk_bert_encode: sequence %d has length %d (1..%d)", b,
                      lens[b], Tmax);
@@ -943,6 +1134,8 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
             tpos.push_back(t);
         }
         rows += lens[b];
+        Lmax = std::max(Lmax, (int) lens[b]);
+        attn_wgs += (int64_t) in.heads * ((lens[b] + BM_Q - 1) / BM_Q);
     }
     const int D = in.hidden, F = in.inter;
     DevGuard guard(m->device);
@@ -1023,9 +1216,13 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
             GSVK_TRY(gemm_q8(m, w.qkv, xq, xqd, rows, 3 * D, D, qkv, nullptr));
         else
             GSVK_TRY(gemm(m, w.qkv, x, x16, x3, rows, 3 * D, D, 1, BgOut{qkv, 0, nullptr, 0, nullptr, nullptr}));
-        hipLaunchKernelGGL(k_bert_attn, dim3((unsigned) ((Tmax + BA_Q - 1) / BA_Q), (unsigned) in.heads, (unsigned) B),
-                           dim3(256), 0, st, qkv, w.qkv_b, d_off, d_len, D, scale_log2, att,
-                           w.ao.f16 ? x16 : nullptr, w3(w.ao) ? x3 : nullptr);
+        uint16_t * a16 = w.ao.f16 ? x16 : nullptr, * a3 = w3(w.ao) ? x3 : nullptr;
+        if (attn_wgs > BERT_ATTN_WGS)
+            hipLaunchKernelGGL(k_bert_attn_mfma, dim3((unsigned) ((Lmax + BM_Q - 1) / BM_Q), (unsigned) in.heads, (unsigned) B),
+                               dim3(256), 0, st, qkv, w.qkv_b, d_off, d_len, D, scale_log2, att, a16, a3);
+        else
+            hipLaunchKernelGGL(k_bert_attn, dim3((unsigned) ((Lmax + BA_Q - 1) / BA_Q), (unsigned) in.heads, (unsigned) B),
+                               dim3(256), 0, st, qkv, w.qkv_b, d_off, d_len, D, scale_log2, att, a16, a3);
         GSVK_LAUNCH_CHECK();
         // out projection (F16 / F32: in K slices when the rows are few; LN1 sums the slices)
         int s1 = 1;
@@ -1060,7 +1257,7 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
     }
     // [rows][D] -> per sequence [D][len], on the device (on the host the strided walk took longer
     // than all kernels: 2,200 rows 6.5 ms)
-    hipLaunchKernelGGL(k_bert_features, dim3((unsigned) ((Tmax + 31) / 32), (unsigned) (D / 32), (unsigned) B), dim3(256),
+    hipLaunchKernelGGL(k_bert_features, dim3((unsigned) ((Lmax + 31) / 32), (unsigned) (D / 32), (unsigned) B), dim3(256),
                        0, st, x, d_off, d_len, D, qkv);
     GSVK_LAUNCH_CHECK();
     GSVK_HIP(hipMemcpyAsync(m->pin, qkv, (size_t) rows * D * 4, hipMemcpyDeviceToHost, st));

@@ -41,6 +41,25 @@ __device__ __forceinline__ void split3(float x, uint16_t & h, uint16_t & m, uint
     l = __builtin_bit_cast(uint16_t, (__bf16) (r - (float) mb));
 }
 
+// The same for a pair of values below 2^127 (an infinity gives NaN in m and l).
+__device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t & h, uint32_t & m, uint32_t & l) {
+    typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+    const auto pk = [](float a, float b) { return __builtin_bit_cast(uint32_t, v2b{(__bf16) a, (__bf16) b}); };
+    const auto lo = [](uint32_t u) { return __builtin_bit_cast(float, u << 16); };
+    const auto hi = [](uint32_t u) { return __builtin_bit_cast(float, u & 0xffff0000u); };
+    h = pk(x0, x1);
+    const float r0 = x0 - lo(h), r1 = x1 - hi(h);
+    m = pk(r0, r1);
+    l = pk(r0 - lo(m), r1 - hi(m));
+}
+
+// The e-th of the six products of a (planes of an operand A) and b (of an operand B), the smallest
+// first; 5 is the large one.
+__device__ __forceinline__ bv16f mfma3(int e, const uint4 (&a)[3], const uint4 (&b)[3], bv16f acc) {
+    constexpr int qa[6] = {0, 2, 1, 0, 1, 0}, qb[6] = {2, 0, 1, 1, 0, 0};
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bv8b, a[qa[e]]), __builtin_bit_cast(bv8b, b[qb[e]]), acc, 0, 0, 0);
+}
+
 // Store N (4 or 8, aligned) consecutive k values of a row as fp16 / as the three planes.
 template <int N>
 __device__ __forceinline__ void store_op16(uint16_t * dst, const float * y) {

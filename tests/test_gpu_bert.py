@@ -126,6 +126,18 @@ def test_tiled_projections(gpu, tmp_path_factory, wtype, lens):
         m.close()
 
 
+@pytest.mark.parametrize("lens", [(32, 31, 33, 1, 64), (127, 128, 129), (257, 2, 96, 160), (512, 1)])
+def test_attention_on_the_matrix_cores(bert_f32, lens):
+    """Key and query tiles with remainders (tiles of 32 keys, 128 queries); the bound of
+    test_tiled_projections."""
+    m, W = bert_f32
+    rng = np.random.default_rng(sum(lens))
+    seqs = [_ids(rng, n) for n in lens]
+    for q, got in zip(seqs, m.encode(seqs)):
+        err = _check(got, BO.encode(W, q, 2, 1024, 16, 1e-12))
+        assert err <= 2e-6, err
+
+
 def test_gsv_bert_class_drop_in(bert_f32, tmp_path_factory):
     """The C++ gsv_bert class (include/gsv_bert.h) through every member, driven by
     tests/dropin/gsv_bert_check.cpp (built by oracle/Makefile, target bertcheck)."""
