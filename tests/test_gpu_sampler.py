@@ -115,3 +115,9 @@ def test_top_k_pivot_against_oracle(gpu, top_k, kind):
         t_ref, s_ref = O.sample(ref, seeds[b])
         assert int(tok.cpu()[b]) == t_ref
         assert int(st.cpu().numpy().view(np.uint64)[b]) == s_ref
+
+
+@pytest.mark.parametrize("top_k", [127, 128, 129, 143, 144, 145, 159, 160, 161, 0])
+def test_survivors_of_one_wave_and_of_four(gpu, top_k):
+    """Up to 128 survivors are one wave's, more are shared by four; the sum reads 32 terms at a time."""
+    test_top_k_pivot_against_oracle(gpu, top_k, "normal")
