@@ -18,9 +18,9 @@
 // and <= 256 VGPRs: 2 workgroups per CU, 2 waves per SIMD). Operands arrive with their quants in
 // natural order (q[row][k]; scales apart). A lane's MFMA operand is one half (16 values) of a
 // block of one row; A and B use the same halves, so the product sums over the block whatever
-// order the hardware assigns to the bytes. Per block a wave issues the MFMA pair of a tile two
-// tiles ahead of the vector work that consumes it, so that the matrix cores and the vector ALUs
-// run side by side.
+// order the hardware assigns to the bytes. A tile's two products are issued one before each half
+// of the vector work on the tile before it, so that the matrix cores and the vector ALUs run side
+// by side also where a SIMD holds one wave (6411 rows x 512 columns, K 2048: 41.3 -> 38.1 us).
 //
 // Epilogue (the options of the decoder's GEMV, layer.h LayerOut): bias, ReLU, fp32 store of
 // columns < n_store, the fp16 K/V append, or the Q8_0 quantisation of each 32-column block (in
@@ -156,9 +156,10 @@ __device__ __forceinline__ void gemm_scales(const GemmOps & o, v8h (&adx)[2], v8
 
 // acc += float(c) * sc over a tile's 16 values per lane (c: exact integer sums of one block; sc:
 // twice the scale products)
+template <int V0>   // half of them
 __device__ __forceinline__ void gemm_fold(float (&acc)[16], const v16i & c, const v16f & sc) {
 #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = __builtin_fmaf((float) c[v], sc[v], acc[v]);
+    for (int v = V0; v < V0 + 8; v++) acc[v] = __builtin_fmaf((float) c[v], sc[v], acc[v]);
 }
 
 // The maximum over each aligned group of 8 lanes, by DPP: quad swaps (1 0 3 2) and (2 3 0 1),
@@ -378,35 +379,35 @@ __global__ void __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu
         // the chunk GM_NBUF - 1 ahead streams into the buffer read before the previous barrier
         if (ch + GM_NBUF - 1 < NCH)
             gemm_issue<NBLK>(xs, xd, ws, wd, io, ch + GM_NBUF - 1, wave, s, (ch + GM_NBUF - 1) % GM_NBUF);
-        GemmOps op = gemm_ops(s, buf, 0, wm, wn, li, lg);
+        GemmOps op[2];
+        op[0] = gemm_ops(s, buf, 0, wm, wn, li, lg);
         v8h adx[2] = {v8h{}, v8h{}}, bdw[2] = {v8h{}, v8h{}};
-        // Per block: the four tiles' MFMA pairs are issued two tiles ahead of the vector work that
-        // consumes them, so that the matrix cores run while the vector ALUs fold the previous
-        // tile; the next block's operands are read from LDS under the last two folds. The
-        // scheduling barriers keep the compiler from regrouping the pairs (it would otherwise
-        // serialise every tile on one result register set).
+        // The 4 tiles of the chunk's blocks as one sequence: under the fold of a tile (32 vector
+        // instructions) the next tile's two products are issued, one before each half of it, so that
+        // neither waits for the matrix cores nor holds up the vector ALUs; the next block's operands
+        // are read from LDS two tiles ahead. The scheduling barriers keep this order.
+        v16i c[2];
+        v16f sc[2];
+        gemm_scales(op[0], adx, bdw);
+        c[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op[0].fa[0], op[0].fb[0], v16i{}, 0, 0, 0);
+        sc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(adx[0], bdw[0], v16f{}, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int bb = 0; bb < GM_KC; bb++) {
-            gemm_scales(op, adx, bdw);
-            const v16i c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(op.fa[0], op.fb[0], v16i{}, 0, 0, 0);
-            const v16f s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(adx[0], bdw[0], v16f{}, 0, 0, 0);
-            const v16i c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(op.fa[0], op.fb[1], v16i{}, 0, 0, 0);
-            const v16f s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(adx[0], bdw[1], v16f{}, 0, 0, 0);
+        for (int it = 0; it < 4 * GM_KC; it++) {
+            const int cur = it & 1, nxt = cur ^ 1, n1 = it + 1;
+            const int ob = (n1 >> 2) & 1, ta = (n1 >> 1) & 1, tb = n1 & 1;   // the next tile's operands
+            if ((it & 3) == 1 && (it >> 2) + 1 < GM_KC) op[((it >> 2) + 1) & 1] = gemm_ops(s, buf, (it >> 2) + 1, wm, wn, li, lg);
+            if (n1 < 4 * GM_KC)
+                c[nxt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op[ob].fa[ta], op[ob].fb[tb], v16i{}, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
-            gemm_fold(acc[0], c0, s0);
+            gemm_fold<0>(acc[it & 3], c[cur], sc[cur]);
             __builtin_amdgcn_sched_barrier(0);
-            const v16i c2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(op.fa[1], op.fb[0], v16i{}, 0, 0, 0);
-            const v16f s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(adx[1], bdw[0], v16f{}, 0, 0, 0);
+            if (n1 < 4 * GM_KC) {
+                if ((n1 & 3) == 0) gemm_scales(op[ob], adx, bdw);
+                sc[nxt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(adx[ta], bdw[tb], v16f{}, 0, 0, 0);
+            }
             __builtin_amdgcn_sched_barrier(0);
-            gemm_fold(acc[1], c1, s1);
-            __builtin_amdgcn_sched_barrier(0);
-            const v16i c3 = __builtin_amdgcn_mfma_i32_32x32x32_i8(op.fa[1], op.fb[1], v16i{}, 0, 0, 0);
-            const v16f s3 = __builtin_amdgcn_mfma_f32_32x32x16_f16(adx[1], bdw[1], v16f{}, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            if (bb + 1 < GM_KC) op = gemm_ops(s, buf, bb + 1, wm, wn, li, lg);
-            __builtin_amdgcn_sched_barrier(0);
-            gemm_fold(acc[2], c2, s2);
-            gemm_fold(acc[3], c3, s3);
+            gemm_fold<8>(acc[it & 3], c[cur], sc[cur]);
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_waitcnt(0);   // the chunks issued so far have landed
