@@ -11,16 +11,17 @@
 // ggml-cpu x86 order (8 lanes, then hsum), so results agree with it to fp32 rounding, not bit
 // for bit; the decode path keeps the bit-exact GEMV.
 //
-// Tiling: workgroup 256 threads = 4 waves, output tile 128 (rows m) x 128 (columns n); wave w
-// owns rows 64*(w/2).. and columns 64*(w%2).., i.e. 2 x 2 MFMA tiles. K is staged through LDS in
-// chunks of 4 blocks (128 values) by direct global -> LDS loads, double buffered: the next
-// chunk streams in while the current one is multiplied, with no staging registers (70 KB of LDS
-// and <= 256 VGPRs: 2 workgroups per CU, 2 waves per SIMD). Operands arrive with their quants in
-// natural order (q[row][k]; scales apart). A lane's MFMA operand is one half (16 values) of a
-// block of one row; A and B use the same halves, so the product sums over the block whatever
-// order the hardware assigns to the bytes. A tile's two products are issued one before each half
-// of the vector work on the tile before it, so that the matrix cores and the vector ALUs run side
-// by side also where a SIMD holds one wave (6411 rows x 512 columns, K 2048: 41.3 -> 38.1 us).
+// Tiling: workgroup 256 threads = 4 waves, output tile 64 MT (rows m) x 128 (columns n), MT = 2 or
+// 1 (gemm_half_tiles); wave w owns rows 32 MT*(w/2).. and columns 64*(w%2).., i.e. MT x 2 MFMA
+// tiles. K is staged through LDS in chunks of 4 blocks (128 values) by direct global -> LDS loads,
+// double buffered: the next chunk streams in while the current one is multiplied, with no staging
+// registers (70 KB of LDS and <= 256 VGPRs: 2 workgroups per CU, 2 waves per SIMD; 52 KB and 3 with
+// MT = 1). Operands arrive with their quants in natural order (q[row][k]; scales apart). A lane's
+// MFMA operand is one half (16 values) of a block of one row; A and B use the same halves, so the
+// product sums over the block whatever order the hardware assigns to the bytes. A tile's two
+// products are issued one before each half of the vector work on the tile before it, so that the
+// matrix cores and the vector ALUs run side by side also where a SIMD holds one wave (6411 rows x
+// 512 columns, K 2048: 41.3 -> 38.1 us with MT = 2, 31.8 us with MT = 1).
 //
 // Epilogue (the options of the decoder's GEMV, layer.h LayerOut): bias, ReLU, fp32 store of
 // columns < n_store, the fp16 K/V append, or the Q8_0 quantisation of each 32-column block (in
@@ -49,19 +50,21 @@ typedef __attribute__((address_space(3))) void lds_void;
 // slot h ^ gemm_swz(r), so that the 16-byte operand reads of a wave (lane (i, g) reads half g of
 // row i) cover every bank once per 8 and per 16 lanes, and every operand address of a wave is
 // one base register plus a constant.
+template <int MT>   // rows of the tile: 64 MT
 struct GemmLds {
-    int8_t a[GM_NBUF][GM_KC][GM_BM][32];
+    int8_t a[GM_NBUF][GM_KC][64 * MT][32];
     int8_t b[GM_NBUF][GM_KC][GM_BN][32];
-    float da[GM_NBUF][GM_BM * GM_KC];      // activation scales [row][block]
+    float da[GM_NBUF][64 * MT * GM_KC];      // activation scales [row][block]
     uint16_t db[GM_NBUF][GM_BN * GM_KC];   // weight scales (fp16) [col][block]
 };
 
 __device__ __forceinline__ int gemm_swz(int r) { return ((r >> 2) ^ (r >> 3)) & 1; }
 
-// The chunk buffers during the K loop; half of the fp32 output tile (64 rows, padded by 4 floats)
+// The chunk buffers during the K loop; 64 rows of the fp32 output tile (padded by 4 floats)
 // in the epilogue.
+template <int MT>
 union GemmSmem {
-    GemmLds k;
+    GemmLds<MT> k;
     float y[GM_BM / 2][GM_BN + 4];
 };
 
@@ -75,23 +78,25 @@ __device__ __forceinline__ void lds_dma4(const void * g, void * lds) {
 // scales travel in pairs)
 
 // Per-lane offsets of a wave's direct loads, fixed over the K loop (32-bit: m * k < 2^31 is
-// checked at launch). Wave w loads rows [32 w, 32 w + 32) of the tile: lane L the half of row
-// 32 w + L / 2 that belongs in its 16-byte LDS slot.
+// checked at launch). Wave w loads weight rows [32 w, 32 w + 32) of the tile: lane L the half of
+// row 32 w + L / 2 that belongs in its 16-byte LDS slot; and activation rows alike (MT = 2), or half
+// of the blocks of rows 32 (w % 2) .. (MT = 1).
+template <int MT>
 struct GemmIssue {
     uint32_t xo, wo;          // quants: row offset + half
-    uint32_t xdo[GM_KC / 2];  // activation scales: 256 (row, block) pairs per instruction
+    uint32_t xdo[MT];         // activation scales: 256 (row, block) pairs per instruction
     uint32_t wdo;             // weight scales: a pair of blocks of one column per lane
 };
 
-template <int NBLK>
-__device__ __forceinline__ GemmIssue gemm_issue_offsets(int m, int m0, int n0, int wave, int lane) {
-    GemmIssue o;
-    const int r = 32 * wave + lane / 2;
-    const uint32_t half = (uint32_t) ((lane & 1) ^ gemm_swz(r));
-    o.xo = (uint32_t) min(m0 + r, m - 1) * (NBLK * 32) + half * 16;
+template <int NBLK, int MT>
+__device__ __forceinline__ GemmIssue<MT> gemm_issue_offsets(int m, int m0, int n0, int wave, int lane) {
+    GemmIssue<MT> o;
+    const int r = 32 * wave + lane / 2, rx = MT == 2 ? r : 32 * (wave & 1) + lane / 2;
+    const uint32_t half = (uint32_t) ((lane & 1) ^ gemm_swz(r));   // (rx and r differ from bit 5 up only)
+    o.xo = (uint32_t) min(m0 + rx, m - 1) * (NBLK * 32) + half * 16 + (MT == 2 ? 0 : (wave >> 1) * (GM_KC / 2) * 32);
     o.wo = (uint32_t) (n0 + r) * (NBLK * 32) + half * 16;
 #pragma unroll
-    for (int u = 0; u < GM_KC / 2; u++) {
+    for (int u = 0; u < MT; u++) {
         const int i = u * 256 + wave * 64 + lane;
         o.xdo[u] = (uint32_t) min(m0 + i / GM_KC, m - 1) * NBLK + i % GM_KC;
     }
@@ -102,18 +107,22 @@ __device__ __forceinline__ GemmIssue gemm_issue_offsets(int m, int m0, int n0, i
 
 // Issue the direct loads of one K chunk into buffer buf. A wave's load instruction writes 64
 // consecutive 16-byte (or 4-byte) LDS slots, lane L the L-th.
-template <int NBLK>
+template <int NBLK, int MT>
 __device__ __forceinline__ void gemm_issue(const int8_t * __restrict__ xs, const float * __restrict__ xd,
                                            const int8_t * __restrict__ ws, const uint16_t * __restrict__ wd,
-                                           const GemmIssue & o, int chunk, int wave, GemmLds & s, int buf) {
+                                           const GemmIssue<MT> & o, int chunk, int wave, GemmLds<MT> & s, int buf) {
     const int blk0 = chunk * GM_KC;
 #pragma unroll
     for (int u = 0; u < GM_KC; u++) {
-        lds_dma16(xs + (blk0 + u) * 32 + o.xo, &s.a[buf][u][32 * wave][0]);
+        if constexpr (MT == 2)
+            lds_dma16(xs + (blk0 + u) * 32 + o.xo, &s.a[buf][u][32 * wave][0]);
+        else if (u < GM_KC / 2)
+            lds_dma16(xs + (blk0 + u) * 32 + o.xo, &s.a[buf][(wave >> 1) * (GM_KC / 2) + u][32 * (wave & 1)][0]);
         lds_dma16(ws + (blk0 + u) * 32 + o.wo, &s.b[buf][u][32 * wave][0]);
     }
+    static_assert(64 * GM_KC == 256, "MT activation-scale loads per wave");
 #pragma unroll
-    for (int u = 0; u < GM_KC / 2; u++) lds_dma4(xd + blk0 + o.xdo[u], &s.da[buf][u * 256 + wave * 64]);
+    for (int u = 0; u < MT; u++) lds_dma4(xd + blk0 + o.xdo[u], &s.da[buf][u * 256 + wave * 64]);
     // 128 columns x GM_KC fp16 scales, two per 4-byte lane: 64 * GM_KC lanes
     static_assert(GM_BN * GM_KC / 2 == 256, "one weight-scale load per wave");
     lds_dma4(wd + blk0 + o.wdo, &s.db[buf][2 * (wave * 64)]);
@@ -121,20 +130,26 @@ __device__ __forceinline__ void gemm_issue(const int8_t * __restrict__ xs, const
 
 // One block's MFMA operands for a wave: 16 quants of each of its two row groups (A) and
 // column groups (B), and the raw scales of those rows and columns (see gemm_scales).
+template <int MT>
 struct GemmOps {
-    v4i fa[2], fb[2];
-    float dx[2];
+    v4i fa[MT], fb[2];
+    float dx[MT];
     uint32_t dw[2];   // fp16 bits
 };
 
-__device__ __forceinline__ GemmOps gemm_ops(const GemmLds & s, int buf, int bb, int wm, int wn, int li, int lg) {
-    GemmOps o;
+template <int MT>
+__device__ __forceinline__ GemmOps<MT> gemm_ops(const GemmLds<MT> & s, int buf, int bb, int wm, int wn, int li, int lg) {
+    GemmOps<MT> o;
+#pragma unroll
+    for (int h = 0; h < MT; h++) {
+        const int ra = wm + 32 * h + li;
+        o.fa[h] = *reinterpret_cast<const v4i *>(&s.a[buf][bb][ra][16 * (lg ^ gemm_swz(li))]);
+        o.dx[h] = s.da[buf][ra * GM_KC + bb];
+    }
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        const int ra = wm + 32 * h + li, rb = wn + 32 * h + li;
-        o.fa[h] = *reinterpret_cast<const v4i *>(&s.a[buf][bb][ra][16 * (lg ^ gemm_swz(li))]);
+        const int rb = wn + 32 * h + li;
         o.fb[h] = *reinterpret_cast<const v4i *>(&s.b[buf][bb][rb][16 * (lg ^ gemm_swz(li))]);
-        o.dx[h] = s.da[buf][ra * GM_KC + bb];
         o.dw[h] = s.db[buf][rb * GM_KC + bb];
     }
     return o;
@@ -146,10 +161,11 @@ __device__ __forceinline__ GemmOps gemm_ops(const GemmLds & s, int buf, int bb, 
 // returns 2 * dx * dw, exactly (both are fp16 values, so dx * dw is exact in fp32 and doubling
 // it is too). The accumulators thus hold exactly twice the sum; the epilogue halves them, which
 // is exact as well.
-__device__ __forceinline__ void gemm_scales(const GemmOps & o, v8h (&adx)[2], v8h (&bdw)[2]) {
+template <int MT>
+__device__ __forceinline__ void gemm_scales(const GemmOps<MT> & o, v8h (&adx)[MT], v8h (&bdw)[2]) {
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        adx[h][0] = (_Float16) o.dx[h];
+        if (h < MT) adx[h][0] = (_Float16) o.dx[h];
         bdw[h][0] = __builtin_bit_cast(_Float16, (uint16_t) o.dw[h]);
     }
 }
@@ -174,6 +190,7 @@ __device__ __forceinline__ float max8_lanes(float v) {
 // The tile of this workgroup. The hardware deals workgroup ids round-robin to the 8 XCDs.
 // Renumbered so that each XCD takes a contiguous run of tiles (column tiles fastest), the column
 // tiles of a row tile run on one XCD and share its L2 copy of the activation rows.
+template <int BM>
 __device__ __forceinline__ void gemm_tile_origin(int n, int & n0, int & m0) {
     const int total = (int) gridDim.x, b = (int) blockIdx.x;
     const int per = (total + 7) / 8, tall = total % 8 == 0 ? 8 : total % 8;
@@ -181,15 +198,16 @@ __device__ __forceinline__ void gemm_tile_origin(int n, int & n0, int & m0) {
     const int t = xcd < tall ? xcd * per + loc : tall * per + (xcd - tall) * (per - 1) + loc;
     const int nx = n / GM_BN;
     n0 = (t % nx) * GM_BN;
-    m0 = (t / nx) * GM_BM;
+    m0 = (t / nx) * BM;
 }
 
 // A tile of left-padding rows only (out.row_pad): zeros out, no products; returns whether the
 // tile was one (the same answer in every thread).
+template <int BM>
 __device__ __forceinline__ bool gemm_pad_tile(const LayerOut & out, int n, int m, int n0, int m0, int tid) {
     bool all_pad = true;
     const int S = out.rows_per_seq;
-    const int mend = min(m0 + GM_BM, m);
+    const int mend = min(m0 + BM, m);
     for (int r0 = m0; r0 < mend && all_pad;) {
         const int b = r0 / S;
         const int e = min((b + 1) * S, mend);
@@ -210,16 +228,17 @@ __device__ __forceinline__ bool gemm_pad_tile(const LayerOut & out, int n, int m
     return true;
 }
 
-// The epilogue of the 128 x 128 GEMMs: acc (a wave's 2 x 2 tiles of 32 x 32) times f is the
-// output tile; yl is the LDS space of half the tile (64 rows, padded by 4 floats).
-__device__ __forceinline__ void gemm_epilogue(float (*yl)[GM_BN + 4], const float (&acc)[4][16], float f,
+// The epilogue of the 64 MT x 128 GEMMs: acc (a wave's MT x 2 tiles of 32 x 32) times f is the
+// output tile; yl is the LDS space of 64 rows of it (padded by 4 floats).
+template <int MT>
+__device__ __forceinline__ void gemm_epilogue(float (*yl)[GM_BN + 4], const float (&acc)[2 * MT][16], float f,
                                               const LayerOut & out, int n, int m, int n0, int m0, int wave,
                                               int lane) {
-    const int wm = (wave >> 1) * 64;
+    const int wm = (wave >> 1) * 32 * MT;
     const int wn = (wave & 1) * 64;
     const int li = lane & 31;
     const int lg = lane >> 5;
-    // Each half of the 128 x 128 tile goes through LDS; then a wave takes 16 of its rows, two per
+    // Each 64 rows of the tile go through LDS; then a wave takes 16 of its rows, two per
     // step, lane l the 4 columns 4 (l % 32).. of row 2 i + l / 32, so that every store instruction
     // writes whole rows (fp32: 512 bytes, Q8_0: 128 bytes, K/V: 64 bytes per head) and a Q8_0
     // block is 8 lanes (its absmax: three exchanges).
@@ -250,15 +269,15 @@ __device__ __forceinline__ void gemm_epilogue(float (*yl)[GM_BN + 4], const floa
         kv_head = (rr / out.d_model == 0 ? out.kc : out.vc) + ((rr % out.d_model) >> 5) * out.lstride * 32 + (col & 31);
     }
 #pragma unroll 1
-    for (int half = 0; half < 2; half++) {
+    for (int half = 0; half < MT; half++) {
         if (half) __syncthreads();       // the first half has been read
-        if (wm == 64 * half) {
+        if (MT == 1 || wm == 64 * half) {
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
+            for (int t = 0; t < 2 * MT; t++) {
                 const int ta = t >> 1, tb = t & 1;
 #pragma unroll
                 for (int v = 0; v < 16; v++)
-                    yl[32 * ta + 8 * (v >> 2) + 4 * lg + (v & 3)][wn + 32 * tb + li] = f * acc[t][v];
+                    yl[(MT == 1 ? wm : 32 * ta) + 8 * (v >> 2) + 4 * lg + (v & 3)][wn + 32 * tb + li] = f * acc[t][v];
             }
         }
         __syncthreads();
@@ -341,35 +360,36 @@ __device__ __forceinline__ void gemm_epilogue(float (*yl)[GM_BN + 4], const floa
     }
 }
 
-template <int NBLK>
+template <int NBLK, int MT>
 __global__ void __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(2))) k_q8_gemm(const int8_t * __restrict__ ws,
                                                            const uint16_t * __restrict__ wd, int n, int m,
                                                            const int8_t * __restrict__ xs,
                                                            const float * __restrict__ xd, LayerOut out) {
     constexpr int NCH = NBLK / GM_KC;
-    __shared__ __align__(16) GemmSmem sm;
-    GemmLds & s = sm.k;
+    constexpr int NT = 2 * MT;         // tiles of a wave
+    __shared__ __align__(16) GemmSmem<MT> sm;
+    GemmLds<MT> & s = sm.k;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     int n0, m0;
-    gemm_tile_origin(n, n0, m0);
-    if (out.row_pad && gemm_pad_tile(out, n, m, n0, m0, tid)) return;   // (uniform)
-    const int wm = (wave >> 1) * 64;   // this wave's rows within the tile
+    gemm_tile_origin<64 * MT>(n, n0, m0);
+    if (out.row_pad && gemm_pad_tile<64 * MT>(out, n, m, n0, m0, tid)) return;   // (uniform)
+    const int wm = (wave >> 1) * 32 * MT;   // this wave's rows within the tile
     const int wn = (wave & 1) * 64;    // and columns
     const int li = lane & 31;          // MFMA: row of A / column of B held by this lane
     const int lg = lane >> 5;          // MFMA: which half of the block
 
-    float acc[4][16];                  // tile t = 2 * ta + tb; twice the output (see gemm_ops)
+    float acc[2 * MT][16];             // tile t = 2 * ta + tb; twice the output (see gemm_ops)
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+    for (int t = 0; t < 2 * MT; t++)
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[t][v] = 0.0f;
 
-    const GemmIssue io = gemm_issue_offsets<NBLK>(m, m0, n0, wave, lane);
+    const GemmIssue<MT> io = gemm_issue_offsets<NBLK, MT>(m, m0, n0, wave, lane);
 #pragma unroll
     for (int c = 0; c < GM_NBUF - 1; c++)
-        if (c < NCH) gemm_issue<NBLK>(xs, xd, ws, wd, io, c, wave, s, c);
+        if (c < NCH) gemm_issue<NBLK, MT>(xs, xd, ws, wd, io, c, wave, s, c);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
@@ -378,11 +398,11 @@ __global__ void __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu
         const int buf = ch % GM_NBUF;
         // the chunk GM_NBUF - 1 ahead streams into the buffer read before the previous barrier
         if (ch + GM_NBUF - 1 < NCH)
-            gemm_issue<NBLK>(xs, xd, ws, wd, io, ch + GM_NBUF - 1, wave, s, (ch + GM_NBUF - 1) % GM_NBUF);
-        GemmOps op[2];
+            gemm_issue<NBLK, MT>(xs, xd, ws, wd, io, ch + GM_NBUF - 1, wave, s, (ch + GM_NBUF - 1) % GM_NBUF);
+        GemmOps<MT> op[2];
         op[0] = gemm_ops(s, buf, 0, wm, wn, li, lg);
-        v8h adx[2] = {v8h{}, v8h{}}, bdw[2] = {v8h{}, v8h{}};
-        // The 4 tiles of the chunk's blocks as one sequence: under the fold of a tile (32 vector
+        v8h adx[MT] = {}, bdw[2] = {};
+        // The wave's tiles of the chunk's blocks as one sequence: under the fold of a tile (32 vector
         // instructions) the next tile's two products are issued, one before each half of it, so that
         // neither waits for the matrix cores nor holds up the vector ALUs; the next block's operands
         // are read from LDS two tiles ahead. The scheduling barriers keep this order.
@@ -393,28 +413,28 @@ __global__ void __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu
         sc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(adx[0], bdw[0], v16f{}, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int it = 0; it < 4 * GM_KC; it++) {
+        for (int it = 0; it < NT * GM_KC; it++) {
             const int cur = it & 1, nxt = cur ^ 1, n1 = it + 1;
-            const int ob = (n1 >> 2) & 1, ta = (n1 >> 1) & 1, tb = n1 & 1;   // the next tile's operands
-            if ((it & 3) == 1 && (it >> 2) + 1 < GM_KC) op[((it >> 2) + 1) & 1] = gemm_ops(s, buf, (it >> 2) + 1, wm, wn, li, lg);
-            if (n1 < 4 * GM_KC)
+            const int ob = (n1 / NT) & 1, ta = (n1 % NT) >> 1, tb = n1 & 1;   // the next tile's operands
+            if (it % NT == MT - 1 && it / NT + 1 < GM_KC) op[(it / NT + 1) & 1] = gemm_ops(s, buf, it / NT + 1, wm, wn, li, lg);
+            if (n1 < NT * GM_KC)
                 c[nxt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op[ob].fa[ta], op[ob].fb[tb], v16i{}, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
-            gemm_fold<0>(acc[it & 3], c[cur], sc[cur]);
+            gemm_fold<0>(acc[it % NT], c[cur], sc[cur]);
             __builtin_amdgcn_sched_barrier(0);
-            if (n1 < 4 * GM_KC) {
-                if ((n1 & 3) == 0) gemm_scales(op[ob], adx, bdw);
+            if (n1 < NT * GM_KC) {
+                if (n1 % NT == 0) gemm_scales(op[ob], adx, bdw);
                 sc[nxt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(adx[ta], bdw[tb], v16f{}, 0, 0, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-            gemm_fold<8>(acc[it & 3], c[cur], sc[cur]);
+            gemm_fold<8>(acc[it % NT], c[cur], sc[cur]);
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_waitcnt(0);   // the chunks issued so far have landed
         __syncthreads();                 // and every wave is done with this one
     }
 
-    gemm_epilogue(sm.y, acc, 0.5f, out, n, m, n0, m0, wave, lane);   // (acc holds twice the output)
+    gemm_epilogue<MT>(sm.y, acc, 0.5f, out, n, m, n0, m0, wave, lane);   // (acc holds twice the output)
 }
 
 // ---- Q8_0 activations x fp16 weights on the fp16 matrix cores (the prefill's fp16 mode) ----
@@ -558,8 +578,8 @@ __global__ void __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu
     const int lane = tid & 63;
     const int wave = tid >> 6;
     int n0, m0;
-    gemm_tile_origin(n, n0, m0);
-    if (out.row_pad && gemm_pad_tile(out, n, m, n0, m0, tid)) return;   // (uniform)
+    gemm_tile_origin<GM_BM>(n, n0, m0);
+    if (out.row_pad && gemm_pad_tile<GM_BM>(out, n, m, n0, m0, tid)) return;   // (uniform)
     const int wm = (wave >> 1) * 64;
     const int wn = (wave & 1) * 64;
     const int li = lane & 31;
@@ -612,7 +632,7 @@ __global__ void __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int v = 0; v < 16; v++) accf[t][v] = acc[t][v];
-    gemm_epilogue(sm.y, accf, 1.0f, out, n, m, n0, m0, wave, lane);
+    gemm_epilogue<2>(sm.y, accf, 1.0f, out, n, m, n0, m0, wave, lane);
 }
 
 // w16[n][k] = fp16(d[n][k/32] * q[n][k]) (nearest even): each thread 16 values
@@ -680,6 +700,15 @@ int launch_q8h_gemm(const uint16_t * w16, int64_t n, int64_t k, int64_t m, const
 // (lane (li, lg): 16 values of row/column li, half lg of the block), a group of blocks ahead of
 // its use. The four partial tiles are summed through LDS in wave order, so the result does not
 // depend on timing. Same arithmetic per block as k_q8_gemm.
+// Number of 128-row tiles below which k_q8_gemm takes 64-row ones: twice the workgroups, three
+// instead of two of them resident on a CU. us, 64-row / 128-row tiles (number of the latter):
+//   K 2048, N  512: 300 rows (12) 19.4 / 30.9, 6411 (204) 31.9 / 35.6, 16384 (512) 57.2 / 57.3, 25600 (800) 94.6 / 100.4
+//   K  512, N  512: 300 rows (12)  9.0 / 12.0, 6411 (204) 12.7 / 13.8, 16384 (512) 21.0 / 21.4, 25600 (800) 32.3 / 36.2
+//   K  512, N 2048: 300 rows (48)  8.6 / 11.6, 6411 (816) 32.4 / 34.1, 10000 (1264) 44.7 / 42.7, 25600 (3200) 100.2 / 99.1
+//   K 1024, N 4096: 600 rows (160) 19.0 / 20.9, 2000 (512) 34.1 / 33.6, 4000 (1024) 65.4 / 61.9
+//   K 4096, N 1024: 600 rows (40) 36.7 / 60.1, 4000 (256) 60.1 / 71.6, 6411 (408) 103.4 / 100.5, 8192 (512) 111.6 / 106.0
+// (the rows of N 1024 and 4096 are the BERT encoder's)
+constexpr int64_t gemm_half_tiles(int64_t k) { return k == 512 || k == 2048 ? 1024 : 384; }
 constexpr int64_t GS_MAX_ROWS = 256;      // launch_q8_gemm takes this kernel up to this many rows
 
 template <int NBLK, int MT, int W = 4>   // W waves, each a W-th of K
@@ -909,15 +938,23 @@ int launch_q8_gemm(const Q8Weights & w, int64_t n, int64_t k, int64_t m, const i
                  "q8_gemm: above %lld rows the operands are in natural order", (long long) GS_MAX_ROWS);
     const int8_t * ws = w.qn;
     const uint16_t * wd = w.dn;
-    const dim3 grid((unsigned) (n / GM_BN * ((m + GM_BM - 1) / GM_BM)));
-    if (k == 512)
-        hipLaunchKernelGGL(k_q8_gemm<16>, grid, dim3(GM_THREADS), 0, stream, ws, wd, (int) n, (int) m, xs, xd, out);
-    else if (k == 1024)
-        hipLaunchKernelGGL(k_q8_gemm<32>, grid, dim3(GM_THREADS), 0, stream, ws, wd, (int) n, (int) m, xs, xd, out);
-    else if (k == 2048)
-        hipLaunchKernelGGL(k_q8_gemm<64>, grid, dim3(GM_THREADS), 0, stream, ws, wd, (int) n, (int) m, xs, xd, out);
-    else
-        hipLaunchKernelGGL(k_q8_gemm<128>, grid, dim3(GM_THREADS), 0, stream, ws, wd, (int) n, (int) m, xs, xd, out);
+    const bool half = n / GM_BN * ((m + GM_BM - 1) / GM_BM) < gemm_half_tiles(k);
+    const int64_t bm = half ? GM_BM / 2 : GM_BM;
+    const dim3 grid((unsigned) (n / GM_BN * ((m + bm - 1) / bm)));
+#define GSVK_GM(NB)                                                                                                \
+    do {                                                                                                           \
+        if (half)                                                                                                  \
+            hipLaunchKernelGGL((k_q8_gemm<NB, 1>), grid, dim3(GM_THREADS), 0, stream, ws, wd, (int) n, (int) m, xs, \
+                               xd, out);                                                                           \
+        else                                                                                                       \
+            hipLaunchKernelGGL((k_q8_gemm<NB, 2>), grid, dim3(GM_THREADS), 0, stream, ws, wd, (int) n, (int) m, xs, \
+                               xd, out);                                                                           \
+    } while (0)
+    if (k == 512) GSVK_GM(16);
+    else if (k == 1024) GSVK_GM(32);
+    else if (k == 2048) GSVK_GM(64);
+    else GSVK_GM(128);
+#undef GSVK_GM
     GSVK_LAUNCH_CHECK();
     return GSVK_OK;
 }

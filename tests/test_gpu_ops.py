@@ -468,6 +468,25 @@ def test_q8_gemm_matches_oracle(gpu, n, k, m):
     assert np.abs(y2.cpu().numpy() - ref2).max() <= 2e-6 * scale
 
 
+@pytest.mark.parametrize("n,k,full", [(2048, 512, 8192), (4096, 1024, 1536), (1024, 4096, 6144)])
+def test_q8_gemm_tile_heights_agree(gpu, n, k, full):
+    """At `full` rows the tiles are 128 high, below 64 (a remainder of 1 to 64 rows in the last one):
+    a row's sums run in the same order, so the same bits."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    ri = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device="cuda", generator=g)  # noqa: E731
+    wq, xq = ri(n, k), ri(full, k)
+    wd = torch.rand(n, k // 32, device="cuda", generator=g).half().view(torch.int16)
+    xd = torch.rand(full, k // 32, device="cuda", generator=g).half().float()
+    y = torch.empty(full, n, device="cuda")
+    gpu.op_q8_gemm(wq, wd, n, k, xq, xd, full, None, 0, y)
+    for m in (1025, 1087, 1088, 1089, 1151, 1152):
+        y2 = torch.full((m + 1, n), 7.0, device="cuda")
+        gpu.op_q8_gemm(wq, wd, n, k, xq[:m].contiguous(), xd[:m].contiguous(), m, None, 0, y2)
+        assert torch.equal(y2[:m], y[:m]), m
+        assert bool((y2[m] == 7.0).all()), m
+
+
 @pytest.mark.parametrize("n,k", [(2048, 512), (512, 2048), (1024, 4096)])
 @pytest.mark.parametrize("m", [300, 1024])
 @pytest.mark.parametrize("with_y", [True, False])
