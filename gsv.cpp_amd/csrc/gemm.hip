@@ -929,12 +929,9 @@ int launch_q8_gemm(const Q8Weights & w, int64_t n, int64_t k, int64_t m, const i
     GSVK_REQUIRE(((uintptr_t) out.bias & 15) == 0 && ((uintptr_t) out.y & 15) == 0 && out.y_stride % 4 == 0 &&
                      ((uintptr_t) out.kc & 15) == 0 && ((uintptr_t) out.vc & 15) == 0,
                  "q8_gemm: bias, y (and its row stride) and the K/V caches must be 16-byte aligned");
-    // A long K over few columns stays with the kernel that splits K over its waves while one workgroup
-    // per CU holds its tiles: the 128-column tiles are too few there, each a chain over all of K.
-    // us, split / tiles: K 2048, N 512: 300 rows 10.1 / 19.4, 700 rows 13.5 / 19.7, 1024 rows 13.7 / 19.7,
-    // 1300 rows 25.2 / 19.9; K 4096, N 1024: 320 rows 23.5 / 34.4, 512 rows 25.7 / 35.9, 640 rows 46.0 / 36.7.
-    const bool split = k >= 2048 && (n / 32) * ((m + 63) / 64) <= 256 && tile_rows == 0;
-    if (m <= GS_MAX_ROWS || split || n % GM_BN != 0 || !w.qn || x_layout == Q8_TILED)
+    // (above GS_MAX_ROWS every row count takes k_q8_gemm, whose order of sums does not depend on it: a
+    // sequence's prefill is then the same bits alone and in a batch)
+    if (m <= GS_MAX_ROWS || n % GM_BN != 0 || !w.qn || x_layout == Q8_TILED)
         return launch_q8_gemm_small(w, n, k, m, xs, xd, x_layout == Q8_TILED, out, tile_rows, stream);
     GSVK_REQUIRE(tile_rows == 0, "q8_gemm: row tiles are a choice of the small-batch kernel (m <= %lld)",
                  (long long) GS_MAX_ROWS);

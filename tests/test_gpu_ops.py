@@ -487,27 +487,6 @@ def test_q8_gemm_tile_heights_agree(gpu, n, k, full):
         assert bool((y2[m] == 7.0).all()), m
 
 
-@pytest.mark.parametrize("n,k,last", [(512, 2048, 1024), (1024, 4096, 512)])
-def test_q8_gemm_long_k_dispatch(gpu, n, k, last):
-    """Up to `last` rows K is split over waves, above the tiles take over: both against the product in
-    64 bits (2e-6 of the scale, as test_q8_gemm_matches_oracle)."""
-    import torch
-    g = torch.Generator(device="cuda").manual_seed(n + k)
-    ri = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device="cuda", generator=g)  # noqa: E731
-    wq, xq = ri(n, k), ri(last + 1, k)
-    wd = torch.rand(n, k // 32, device="cuda", generator=g).half()
-    xd = torch.rand(last + 1, k // 32, device="cuda", generator=g).half()
-    b = torch.randn(n, device="cuda", generator=g)
-    deq = lambda q, d: (q.double().reshape(q.shape[0], -1, 32) * d.double()[..., None]).reshape(q.shape)  # noqa: E731
-    ref = deq(xq, xd) @ deq(wq, wd).T.contiguous() + b.double()
-    for m in (257, 289, last // 2, last // 2 + 1, last, last + 1):
-        y = torch.full((m + 1, n), 7.0, device="cuda")
-        gpu.op_q8_gemm(wq, wd.view(torch.int16), n, k, xq[:m].contiguous(), xd[:m].float().contiguous(), m, b, 0, y)
-        err = ((y[:m].double() - ref[:m]).abs().max() / ref.abs().max()).item()
-        assert err <= 2e-6, (m, err)
-        assert bool((y[m] == 7.0).all()), m
-
-
 @pytest.mark.parametrize("n,k", [(2048, 512), (512, 2048), (1024, 4096)])
 @pytest.mark.parametrize("m", [300, 1024])
 @pytest.mark.parametrize("with_y", [True, False])
