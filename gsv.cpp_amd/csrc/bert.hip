@@ -875,10 +875,11 @@ int load_ln(gsvk_bert * m, const GgufFile & g, const std::string & wn, const std
 // Rows above which the LDS-tiled GEMM takes the projections; at most these the direct loads, which
 // put every weight's load in flight at once. Whole encode of one sequence, us, direct / tiled:
 //   F16  64 rows 825 / 1316, 256 rows 1403 / 1750, 384 rows 1870 / 2060, 512 rows 2105 / 2215;
-//        2265 rows (16 sequences) 5330 / 4845
+//        of several: 2 x 257 rows 2107 / 2038, 6 x 120 2102 / 2135, 8 x 128 2419 / 2494,
+//        3 x 290 2515 / 2448, 4 x 300 3049 / 2868, 16 x 128 3895 / 3539
 //   F32  64 rows 1257 / 1702, 96 rows 1836 / 1792, 128 rows 1855 / 1834, 160 rows 2845 / 2055,
 //        512 rows 5103 / 3425
-// (the F16 lines meet near 600 rows, the F32 lines near 90; the step at 128 -> 160 is a third row tile)
+// (the F16 lines run together from 512 to 1024 rows and part above; the F32 lines meet near 90)
 constexpr int64_t BERT_DIRECT_ROWS_F16 = 512;
 constexpr int64_t BERT_DIRECT_ROWS_F32 = 96;
 bool bert_lds(const Proj & w, int64_t M) { return M > (w.f16 ? BERT_DIRECT_ROWS_F16 : BERT_DIRECT_ROWS_F32); }
