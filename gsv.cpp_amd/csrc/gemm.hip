@@ -756,8 +756,8 @@ __global__ void __launch_bounds__(W * 64) k_q8_gemm_small(Q8Weights w, int n, in
     const float * xdr[MT];
 #pragma unroll
     for (int t = 0; t < MT; t++) {
-        if (x_tiled) {                                  // rows are padded to the tile
-            const int64_t tile = (m0 >> 5) + t;
+        if (x_tiled) {   // rows are padded to the tile; tiles past the last (unused) repeat it
+            const int64_t tile = min((m0 >> 5) + t, (m - 1) >> 5);
             xrow[t] = xs + ((tile * NBLK) << 10) + lane * 16;
             xdr[t] = xd + ((tile * NBLK) << 5) + li;
         } else {

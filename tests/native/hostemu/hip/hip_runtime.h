@@ -18,6 +18,7 @@
 #define __constant__
 #define __forceinline__ inline
 #define __launch_bounds__(...)
+#define amdgpu_waves_per_eu(...) annotate("")   // (an attribute of kernels)
 #define __align__(n) __attribute__((aligned(n)))
 #define __shared__ static
 
@@ -127,6 +128,48 @@ inline int __builtin_amdgcn_sdot4(int a, int b, int c, bool) {
     for (int i = 0; i < 4; i++) s += (int) (int8_t) (a >> (8 * i)) * (int) (int8_t) (b >> (8 * i));
     return s;
 }
+
+inline unsigned __builtin_amdgcn_perm(unsigned a, unsigned b, unsigned sel) {   // (selectors 0..7 only)
+    const uint64_t v = ((uint64_t) a << 32) | b;
+    unsigned r = 0;
+    for (int i = 0; i < 4; i++) r |= (unsigned) ((v >> (8 * ((sel >> (8 * i)) & 7))) & 0xff) << (8 * i);
+    return r;
+}
+
+// ---- matrix instructions: lane 32 g + i holds row (A) / column (B) i's K values [KL g, KL g + KL) of
+// the 2 KL of the product, and of the result column i of the rows 8 (v / 4) + 4 g + v % 4. Every lane
+// publishes its operands, all wait, each sums its 16 outputs, all wait again. ----
+template <typename E, int KL, typename A, typename C>
+inline C emu_mfma_32x32(A a, A b, C c) {
+    static E s_a[16][64][KL], s_b[16][64][KL];
+    static_assert(sizeof(A) == KL * sizeof(E), "operand size");
+    const int lane = (int) (threadIdx.x & 63), wave = (int) (threadIdx.x >> 6);
+    std::memcpy(s_a[wave][lane], &a, sizeof a);
+    std::memcpy(s_b[wave][lane], &b, sizeof b);
+    ::emu::wave_sync();
+    for (int v = 0; v < 16; v++) {
+        const int row = 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3), col = lane & 31;
+        auto s = c[v];
+        for (int g = 0; g < 2; g++)
+            for (int k = 0; k < KL; k++)
+                s += (decltype(s)) s_a[wave][32 * g + row][k] * (decltype(s)) s_b[wave][32 * g + col][k];
+        c[v] = s;
+    }
+    ::emu::wave_sync();
+    return c;
+}
+template <typename A, typename C>
+inline C __builtin_amdgcn_mfma_i32_32x32x32_i8(A a, A b, C c, int, int, int) { return emu_mfma_32x32<int8_t, 16>(a, b, c); }
+template <typename A, typename C>
+inline C __builtin_amdgcn_mfma_f32_32x32x16_f16(A a, A b, C c, int, int, int) { return emu_mfma_32x32<_Float16, 8>(a, b, c); }
+
+// ---- direct global -> LDS loads: lane L's bytes to lds + L * size, at once (a wait that is missing
+// is not seen here) ----
+inline void __builtin_amdgcn_global_load_lds(const void * g, __attribute__((address_space(3))) void * lds, int size, int, int) {
+    std::memcpy((char *) lds + (threadIdx.x & 63) * size, g, size);
+}
+// (a kernel with this barrier in asm assembles, but is not run here)
+asm(".macro s_barrier\n.endm");
 
 // ---- atomics (one fiber runs at a time) ----
 // (__hip_atomic_load / store / fetch_add are clang builtins on the host too; the scopes are not

@@ -630,6 +630,13 @@ def test_q8_gemm_small_tiles(gpu, n, k, m):
     assert np.array_equal(yqt.cpu().numpy(), qt_ref) and np.array_equal(ydt.cpu().numpy(), dt_ref)
 
 
+@pytest.mark.parametrize("n,k,m", [(2048, 512, 160), (1536, 512, 224)])
+def test_q8_gemm_small_tiles_odd_count(gpu, n, k, m):
+    """Two row tiles per workgroup and an odd number of them: the decode's FFN1 from batch 129 and
+    QKV from batch 193."""
+    test_q8_gemm_small_tiles(gpu, n, k, m)
+
+
 @pytest.mark.parametrize("B,S,max_len,pads,what", [
     (3, 300, 100, [0, 17, 60], "text + causal semantic rows, left pads, ragged last tile"),
     (1, 64, 64, [5], "text rows only"),

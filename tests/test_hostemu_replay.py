@@ -67,3 +67,20 @@ def test_exact_fused_kernel_equals_the_two_launches(replay, args):
     r = subprocess.run([CHECK] + [str(a) for a in args], capture_output=True, text=True, env=env, timeout=900)
     assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
     assert "equal to the bit" in r.stdout
+
+
+GEMM = os.path.join(ROOT, "_build", "hostemu", "gemm_check")
+
+
+@pytest.mark.parametrize("n,k,m,tile_rows", [
+    (2048, 512, 160, 0), (1536, 512, 224, 0),      # the decode's FFN1 and QKV at an odd number of row tiles
+    (512, 512, 33, 2), (512, 512, 65, 2), (512, 512, 1, 4), (512, 512, 160, 4), (512, 2048, 96, 4),
+    (1024, 512, 289, 0),                           # tiled activations above 256 rows
+])
+def test_q8_gemm_in_bounds(replay, n, k, m, tile_rows):
+    """The Q8_0 GEMM on buffers of exactly the callers' sizes: with several row tiles of 32 per
+    workgroup the last one may hold tiles past the activations' rows, which are not read."""
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0")
+    r = subprocess.run([GEMM] + [str(a) for a in (n, k, m, tile_rows)], capture_output=True, text=True, env=env,
+                       timeout=900)
+    assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
