@@ -920,18 +920,12 @@ int bert_row_tiles(int64_t M, int N) {
     return M > 32 && (int64_t) (N / BG_BN) * ((M + 63) / 64) >= 256 ? 2 : 1;
 }
 
-// K slices for an [M][N][K] projection: enough workgroups (tiles x slices) to cover the chip when the
-// tiles are few, each slice a multiple of what the kernel takes at a time. Tiled F32: two workgroups
-// per CU (564 rows, FFN2: 4 slices 33 us, 8 slices 31.5, which the LayerNorm's reads give back).
-int bert_kslices(const Proj & w, int64_t M, int N, int K, int max_slices) {
-    if (bert_lds(w, M)) {
-        const BgTile t = bert_tile(w.f16, M, N);
-        const int64_t tiles = (M + t.bm - 1) / t.bm * (N / t.bn);
-        int p = 1;
-        while (p < max_slices && tiles * p < (w.f16 ? 256 : 512) && K % (2 * p * 16 * t.ks) == 0) p *= 2;
-        return p;
-    }
-    const int kmult = BG_WAVES * BG_U * (w.f16 ? BgStep<_Float16>::K : BgStep<float>::K);
+// K values that a workgroup of the direct-load GEMM takes at a time, and its K slices for an
+// [M][N][K] projection: enough workgroups (tiles x slices) to cover the chip when the tiles are few,
+// each slice a multiple of those.
+int bert_kmult(const Proj & w) { return BG_WAVES * BG_U * (w.f16 ? BgStep<_Float16>::K : BgStep<float>::K); }
+int bert_kslices_direct(const Proj & w, int64_t M, int N, int K, int max_slices) {
+    const int kmult = bert_kmult(w);
     const int bm = 32 * bert_row_tiles(M, N);
     const int64_t tiles = (int64_t) (N / BG_BN) * ((M + bm - 1) / bm);
     int p = 1;
@@ -939,16 +933,36 @@ int bert_kslices(const Proj & w, int64_t M, int N, int K, int max_slices) {
     return p;
 }
 
+// The same for the GEMM that takes the projection. Tiled F32: two workgroups per CU (564 rows, FFN2:
+// 4 slices 33 us, 8 slices 31.5, which the LayerNorm's reads give back).
+int bert_kslices(const Proj & w, int64_t M, int N, int K, int max_slices) {
+    if (!bert_lds(w, M)) return bert_kslices_direct(w, M, N, K, max_slices);
+    const BgTile t = bert_tile(w.f16, M, N);
+    const int64_t tiles = (M + t.bm - 1) / t.bm * (N / t.bn);
+    int p = 1;
+    while (p < max_slices && tiles * p < (w.f16 ? 256 : 512) && K % (2 * p * 16 * t.ks) == 0) p *= 2;
+    return p;
+}
+
+constexpr int BERT_MAX_SLICES = 8;   // K slices of the out projection and FFN2
+
 // Y = X . W^T for W of the projection's type (W F16: X16 holds the activations already rounded by
 // their producer; W F32: X, or over many rows their planes X3); `slices` K slices (> 1: partial
 // rows at Y + z * M * N, bias / GELU / y16 not allowed).
 int gemm(gsvk_bert * m, const Proj & W, const float * X, const uint16_t * X16, const uint16_t * X3, int64_t M, int N,
          int K, int slices, const BgOut & o) {
-    const int kmult = BG_WAVES * BG_U * (W.f16 ? BgStep<_Float16>::K : BgStep<float>::K);
+    const int kmult = bert_kmult(W);
     GSVK_REQUIRE(M > 0 && M < (1 << 30) && slices >= 1 &&
                      (slices == 1 || (!o.bias && !o.gelu && !o.y16 && !o.y3)) && (o.y || o.y16 || o.y3),
                  "bert gemm: unsupported shape M=%lld N=%d K=%d slices %d", (long long) M, N, K, slices);
-    if (bert_lds(W, M)) {
+    // groups of steps per wave of the direct loads, which are unrolled. The tiled GEMM takes the same K
+    // (it could take others), so that a file's projections are not refused for some row counts only.
+    const bool lds = bert_lds(W, M);
+    const int ds = lds ? bert_kslices_direct(W, M, N, K, BERT_MAX_SLICES) : slices;
+    const int ng = K / ds / kmult;
+    GSVK_REQUIRE(K % (ds * kmult) == 0 && (ng == 1 || ng == 2 || ng == 4 || ng == 8 || ng == 16),
+                 "bert gemm: K %d / %d slices gives %d groups per wave (1, 2, 4, 8 or 16)", K, ds, ng);
+    if (lds) {
         if (!W.f16) {
             GSVK_REQUIRE(X3 && W.w3, "bert gemm: F32 weights over many rows need the planes");
             return launch_bert_lds<3, 1, 1, 2, 2, 1, 4>(m, X3, W.w3, M, N, K, slices, o);
@@ -959,13 +973,9 @@ int gemm(gsvk_bert * m, const Proj & W, const float * X, const uint16_t * X16, c
             return launch_bert_lds<1, 2, 2, 2, 2, 2, 3>(m, X16, w16, M, N, K, slices, o);
         return launch_bert_lds<1, 1, 2, 2, 2, 4, 3>(m, X16, w16, M, N, K, slices, o);
     }
-    GSVK_REQUIRE(N % BG_BN == 0 && K % (slices * kmult) == 0,
-                 "bert gemm: unsupported shape M=%lld N=%d K=%d slices %d", (long long) M, N, K, slices);
+    GSVK_REQUIRE(N % BG_BN == 0, "bert gemm: unsupported shape M=%lld N=%d K=%d slices %d", (long long) M, N, K, slices);
     const int rt = bert_row_tiles(M, N);
     const dim3 grid((unsigned) (N / BG_BN), (unsigned) ((M + 32 * rt - 1) / (32 * rt)), (unsigned) slices);
-    const int ng = K / slices / kmult;   // groups of steps per wave
-    GSVK_REQUIRE(ng == 1 || ng == 2 || ng == 4 || ng == 8 || ng == 16,
-                 "bert gemm: K %d / %d slices gives %d groups per wave (1, 2, 4, 8 or 16)", K, slices, ng);
 #define GSVK_BG(TT, NGV, XP, WP)                                                                          \
     do {                                                                                                  \
         if (rt == 2)                                                                                      \
@@ -1143,7 +1153,6 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
     hipStream_t st = m->stream;
     // workspace: x, qkv, attention output, projection output (up to BERT_MAX_SLICES partial
     // rows), FFN hidden, the fp16 GEMM inputs (a D-wide row, the FFN hidden), the small arrays
-    constexpr int BERT_MAX_SLICES = 8;
     const size_t fl = (size_t) rows * (D + 3 * D + D + (size_t) BERT_MAX_SLICES * D + F);
     const int64_t rowsp = (rows + BG_ROW_PAD - 1) / BG_ROW_PAD * BG_ROW_PAD;   // rows of the operand order
     const size_t n16 = m->any_f16 ? (size_t) rowsp * (D + F) : 0;

@@ -138,6 +138,22 @@ def test_attention_on_the_matrix_cores(bert_f32, lens):
         assert err <= 2e-6, err
 
 
+@pytest.mark.parametrize("wtype,rows", [("f16", (40, 512, 600)), ("f32", (40, 96, 200))])
+def test_refused_ffn_width_is_refused_at_every_row_count(gpu, tmp_path, wtype, rows):
+    """The direct-load GEMM's loop exists for 1 to 16 groups of steps in powers of two; FFN 1536 (3 or 6
+    groups) is refused also where the tiled GEMM takes the rows."""
+    path, _ = sm.write_bert_model(str(tmp_path / "b.gguf"), n_layer=1, layers_used=1, hidden=512, heads=8, inter=1536,
+                                  vocab=100, wtype=wtype)
+    m = gsvk.Bert(path)
+    try:
+        for n in rows:
+            seqs = [np.zeros(min(512, n - i), np.int32) for i in range(0, n, 512)]
+            with pytest.raises(gsvk.GsvkError, match="groups per wave"):
+                m.encode(seqs)
+    finally:
+        m.close()
+
+
 def test_gsv_bert_class_drop_in(bert_f32, tmp_path_factory):
     """The C++ gsv_bert class (include/gsv_bert.h) through every member, driven by
     tests/dropin/gsv_bert_check.cpp (built by oracle/Makefile, target bertcheck)."""
