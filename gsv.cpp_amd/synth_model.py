@@ -231,12 +231,13 @@ def synth_requests(seed: int, B: int, prompt_len: int, phone_lens, bert: bool = 
 
 def write_bert_model(path: str, seed: int = 0x6A5E0010, n_layer: int = 4, layers_used: int = 2,
                      hidden: int = 1024, heads: int = 16, inter: int = 4096, vocab: int = 1000,
-                     max_pos: int = 512, wtype: str = "f32", ln_eps: float = 1e-12):
+                     max_pos: int = 512, wtype="f32", ln_eps: float = 1e-12, edit=None):
     """A synthetic BERT GGUF with the tensor contract of src/gsv_bert.cpp:398-431 (keys bert.*,
     tensors bert.word_emb .. bert.l{i}.out_ln_b; projection weights in `wtype`, the rest F32, as
     tools/export_gguf/convert_bert.py writes them). Returns (path, weights): the fp32 values the
     loader holds (F16 rounded, Q8_0 dequantised; for Q8_0 also the blocks, under name + "#q8"),
-    for the oracle."""
+    for the oracle. `wtype`: f32, f16 or q8_0, or a function of the projection's name; `edit`
+    (name, values) may replace a tensor's values."""
     rng = np.random.Generator(np.random.PCG64(seed))
     D, F = hidden, inter
 
@@ -259,11 +260,14 @@ def write_bert_model(path: str, seed: int = 0x6A5E0010, n_layer: int = 4, layers
     W = {}
 
     def add(name, a, proj=False):
-        if proj and wtype == "f16":
+        t = (wtype(name) if callable(wtype) else wtype) if proj else "f32"
+        if edit:
+            a = np.asarray(edit(name, a), np.float32)
+        if t == "f16":
             h = a.astype(np.float16)
             w.add_tensor(name, a.shape, GGML_F16, h.tobytes())
             W[name] = h.astype(np.float32)
-        elif proj and wtype == "q8_0":
+        elif t == "q8_0":
             blocks = q8_quantize_ref(a)
             w.add_tensor(name, a.shape, GGML_Q8_0, blocks.tobytes())
             W[name] = q8_dequant(blocks, a.shape[-1]).reshape(a.shape)

@@ -81,11 +81,12 @@ def q8_matmul(x: np.ndarray, blocks: np.ndarray, n: int, k: int) -> np.ndarray:
     return np.einsum("mnb,mb,nb->mn", s.astype(np.float64), dx, dw)
 
 
-def encode(W: dict, ids, n_layers: int, hidden: int, heads: int, eps: float, act_f16: bool = False,
+def encode(W: dict, ids, n_layers: int, hidden: int, heads: int, eps: float, act_f16=False,
            act_q8: bool = False) -> np.ndarray:
     """One sequence of token ids -> [hidden][T] after n_layers layers (0: the embedding LN).
     act_f16: the projections' inputs are rounded to fp16 first, as ggml-cpu does for F16 weights
-    (their vec_dot type is F16: ggml_cpu_fp32_to_fp16 of the activations, then F16 x F16 dots).
+    (their vec_dot type is F16: ggml_cpu_fp32_to_fp16 of the activations, then F16 x F16 dots); a
+    function of the projection's name where a file holds both types.
     act_q8: Q8_0 weights (W holds their blocks under name + "#q8"), multiplied as ggml-cpu does:
     activations quantised to Q8_0 (x86), exact integer block dots (q8_matmul)."""
     ids = np.asarray(ids, np.int64)
@@ -95,13 +96,14 @@ def encode(W: dict, ids, n_layers: int, hidden: int, heads: int, eps: float, act
     x = (g("bert.word_emb")[ids] + g("bert.pos_emb")[:T]) + g("bert.type_emb")[0]
     x = layernorm(x, g("bert.emb_ln_w"), g("bert.emb_ln_b"), eps)
     scale = 1.0 / math.sqrt(hd)
-    r = (lambda a: a.astype(np.float32).astype(np.float16).astype(np.float64)) if act_f16 else (lambda a: a)
+    r16 = lambda a: a.astype(np.float32).astype(np.float16).astype(np.float64)
+    is16 = act_f16 if callable(act_f16) else lambda name: act_f16
 
     def mm(a, name):   # a . W^T of the projection `name`
         if act_q8:
             n_, k_ = W[name].shape
             return q8_matmul(a, W[name + "#q8"], n_, k_)
-        return r(a) @ g(name).T
+        return (r16(a) if is16(name) else a) @ g(name).T
 
     for li in range(n_layers):
         p = f"bert.l{li}."

@@ -126,16 +126,137 @@ def test_tiled_projections(gpu, tmp_path_factory, wtype, lens):
         m.close()
 
 
-@pytest.mark.parametrize("lens", [(32, 31, 33, 1, 64), (127, 128, 129), (257, 2, 96, 160), (512, 1)])
-def test_attention_on_the_matrix_cores(bert_f32, lens):
-    """Key and query tiles with remainders (tiles of 32 keys, 128 queries); the bound of
-    test_tiled_projections."""
-    m, W = bert_f32
-    rng = np.random.default_rng(sum(lens))
-    seqs = [_ids(rng, n) for n in lens]
-    for q, got in zip(seqs, m.encode(seqs)):
-        err = _check(got, BO.encode(W, q, 2, 1024, 16, 1e-12))
-        assert err <= 2e-6, err
+def _mfma_wgs(lens, heads=16):
+    """Workgroups of the matrix-core attention, which is taken above 64 of them."""
+    return heads * sum((n + 127) // 128 for n in lens)
+
+
+# An encoder of one layer whose output is the attention's, so that its error stands alone: every
+# projection one power of two per row (exact in fp32 and in three bf16 planes), FFN zero, LayerNorms
+# without weights. q = 4 x, k = x turned by one dim of the head, v = x / 4 + b, b = +-2 (values of one
+# size, keys weighted unequally), out projection 64: x1 = LN(x + 64 a), output LN(x1).
+KQ, KV, KO = 4.0, 0.25, 64.0
+K_TURN = np.arange(1024) // 64 * 64 + (np.arange(1024) + 1) % 64
+V_BIAS = 2.0 * np.random.default_rng(7).choice([-1.0, 1.0], 1024)
+
+
+def _attention_model(name, a):
+    if ".l0." not in name:
+        return a
+    a = np.zeros_like(a)
+    i = np.arange(1024)
+    if name.endswith("qkv_w"):
+        a[i, i], a[1024 + i, K_TURN], a[2048 + i, i] = KQ, 1.0, KV
+    elif name.endswith("qkv_b"):
+        a[2048:] = V_BIAS
+    elif name.endswith("attn_out_w"):
+        a[i, i] = KO
+    elif name.endswith("ln_w"):
+        a[:] = 1.0
+    return a
+
+
+def _attention_reference(x, drop=None):
+    """The layer on rows x in float64. drop: (which product, "score" or "sum"; the plane pairs left out),
+    the operands then as bf16 planes h + m + l."""
+    import torch
+    one, zero = np.ones(1024), np.zeros(1024)
+
+    def planes(t):
+        out = {}
+        for p in "hml":
+            out[p] = torch.from_numpy(t.astype(np.float32)).bfloat16().double().numpy()
+            t = t - out[p]
+        return out
+
+    def mul(a, b, what):
+        if drop is None or drop[0] != what:
+            return a @ b
+        pa, pb = planes(a.astype(np.float32).astype(np.float64)), planes(b)
+        return sum(pa[e[0]] @ pb[e[1]] for e in ("hh", "hm", "mh", "mm", "hl", "lh") if e not in drop[1])
+
+    v = (KV * x + V_BIAS).astype(np.float32).astype(np.float64)
+    a = np.empty_like(x)
+    for h in range(16):
+        sl = slice(64 * h, 64 * h + 64)
+        s = mul(KQ * x[:, sl], x[:, K_TURN[sl]].T, "score") / 8
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        a[:, sl] = mul(p, v[:, sl], "sum") / p.sum(axis=1, keepdims=True)
+    return BO.layernorm(BO.layernorm(x + KO * a, one, zero, 1e-12), one, zero, 1e-12)
+
+
+# Of the largest output. fp32: scores up to 16, rounded at 2^-24 of that where they enter the exponent,
+# move a weight by 1e-6, of which an output averages several (measured: at most 6.0e-7). A plane product
+# left out: 2^-9 x 2^-9 (mm) or 2^-18 (hl, lh) of a product, rounded planes; 1.5e-6 to 5e-6 here.
+ATTN_TOL = 1e-6
+
+
+@pytest.mark.parametrize("lens", [(32, 31, 33, 1, 64), (127, 128, 129, 1), (257, 2, 96, 160), (512, 1), (128, 64, 200, 3),
+                                  (32, 31, 1, 2, 30)])   # (96 rows in all: plain rows for the direct-load GEMM)
+def test_attention_on_the_matrix_cores(gpu, tmp_path, lens):
+    """Key and query tiles with remainders (tiles of 32 keys, 128 queries), at fp32's precision: the
+    reference with any one of the six plane products left out misses the bound."""
+    assert _mfma_wgs(lens) > 64
+    path, _ = sm.write_bert_model(str(tmp_path / "b.gguf"), n_layer=1, layers_used=1, vocab=1000, edit=_attention_model)
+    m = gsvk.Bert(path)
+    try:
+        rng = np.random.default_rng(sum(lens))
+        seqs = [_ids(rng, n) for n in lens]
+        worst = 0.0
+        for x0, got in zip(m.encode(seqs, n_layers=0), m.encode(seqs)):
+            x = x0.T.astype(np.float64)
+            ref = _attention_reference(x)
+            top = np.abs(ref).max()
+            worst = max(worst, np.abs(got.T - ref).max() / top)
+            if len(x) == 128:
+                for what in ("score", "sum"):
+                    for e in ("mm", "hl", "lh"):
+                        d = np.abs(_attention_reference(x, (what, (e,))) - ref).max() / top
+                        assert d > 1.3 * ATTN_TOL, (what, e, d)
+        print(f"attention {lens}: {worst:.1e}")
+        assert worst <= ATTN_TOL, worst
+    finally:
+        m.close()
+
+
+def test_attention_on_the_matrix_cores_q8_0(gpu, tmp_path_factory):
+    """A Q8_0 batch: the kernel stores plain fp32 rows, which are then quantised. Against one-by-one
+    calls (the other attention kernel): a last-bit difference moves a row where it flips one of its 6144
+    quants after the attention, as in test_quantised_weight_files (a flip before it would move every row
+    of the sequence, but the rows that enter the attention are quantised alike)."""
+    lens = (90, 33, 64, 47, 128)
+    assert _mfma_wgs(lens) > 64 and _mfma_wgs(lens[-1:]) <= 64
+    m, W = _model(tmp_path_factory, "q8_0", 2, 1)
+    try:
+        rng = np.random.default_rng(9)
+        seqs = [_ids(rng, n) for n in lens]
+        rows = []
+        for q, got in zip(seqs, m.encode(seqs)):
+            one = m.encode([q])[0]
+            rows.append(np.abs(got - one).max(axis=0) / np.abs(one).max())
+        row = np.concatenate(rows)
+        print(f"Q8_0 batch: median row {np.median(row):.1e}, {np.sum(row > 1e-4)} of {len(row)} moved, worst {row.max():.1e}")
+        assert np.median(row) <= 1e-5 and np.mean(row > 1e-4) <= 0.1 and row.max() <= 5e-3
+    finally:
+        m.close()
+
+
+@pytest.mark.parametrize("lens", [(40,), (96, 104), (300, 301)])   # both direct, F32 tiled, both tiled
+@pytest.mark.parametrize("hidden", [512, 1024])
+@pytest.mark.parametrize("f16", [("qkv_w", "ff1_w"), ("attn_out_w", "ff2_w")])
+def test_layer_of_mixed_projection_types(gpu, tmp_path, f16, hidden, lens):
+    """F16 and F32 projections in one layer: each producer writes the operand that its consumer takes."""
+    is16 = lambda name: name.endswith(f16)  # noqa: E731
+    path, W = sm.write_bert_model(str(tmp_path / "b.gguf"), n_layer=1, layers_used=1, hidden=hidden, heads=hidden // 64,
+                                  inter=2048, vocab=1000, wtype=lambda n: "f16" if is16(n) else "f32")
+    m = gsvk.Bert(path)
+    try:
+        rng = np.random.default_rng(hidden + sum(lens))
+        seqs = [_ids(rng, n) for n in lens]
+        for q, got in zip(seqs, m.encode(seqs)):
+            _check(got, BO.encode(W, q, 1, hidden, hidden // 64, 1e-12, act_f16=is16))
+    finally:
+        m.close()
 
 
 @pytest.mark.parametrize("wtype,rows", [("f16", (40, 512, 600)), ("f32", (40, 96, 200))])
