@@ -82,7 +82,7 @@ def test_longest_sequence_and_limits(bert_f32):
 def test_quantised_weight_files(gpu, tmp_path_factory, wtype, T):
     """F16 weights: the activations rounded to fp16 before each projection; Q8_0 weights: the
     activations quantised to Q8_0 (x86) and multiplied on the int8 GEMM with exact block sums;
-    both as ggml-cpu does, the oracle likewise. 300 tokens take the 128 x 128 int8 kernel."""
+    both as ggml-cpu does, the oracle likewise. 300 tokens take the int8 kernel of more than 256 rows."""
     m, W = _model(tmp_path_factory, wtype, 2, 1)
     try:
         assert m.info["weight_type"] == (1 if wtype == "f16" else 8)

@@ -78,7 +78,7 @@ def test_kv_write_layer0_bitexact_without_bert(models):
 
 
 @pytest.mark.parametrize("lens,what", [
-    ([260, 300, 245], "128 x 128 tiles: S = 316, 948 rows; alone: 261 rows and more"),
+    ([260, 300, 245], "128-column tiles: S = 316, 948 rows; alone: 261 rows and more"),
     ([70, 100], "32-column tiles, K split over 4 waves: S = 116, 232 rows; alone: 86 and 116 rows"),
 ])
 def test_prefill_on_matrix_cores(models, lens, what):
@@ -87,7 +87,7 @@ def test_prefill_on_matrix_cores(models, lens, what):
     within one fp16 ulp of the oracle's (the fp32 values differ by rounding, which can move a
     value across an fp16 rounding boundary), and left padding changes nothing as long as the
     batch and the request alone fall in the same row range of the GEMM (up to 256 rows: the
-    32-column kernel sums 4 K quarters, above: the 128 x 128 kernel accumulates through K)."""
+    32-column kernel sums 4 K quarters, above: the 128-column one accumulates through K)."""
     g, o = models
     reqs = _reqs(11, lens)
     got = g.first_logits(reqs)

@@ -468,7 +468,7 @@ def test_q8_gemm_matches_oracle(gpu, n, k, m):
     assert np.abs(y2.cpu().numpy() - ref2).max() <= 2e-6 * scale
 
 
-@pytest.mark.parametrize("n,k,full", [(2048, 512, 8192), (4096, 1024, 1536), (1024, 4096, 6144)])
+@pytest.mark.parametrize("n,k,full", [(2048, 512, 8192), (512, 2048, 32768), (4096, 1024, 1536), (1024, 4096, 6144)])
 def test_q8_gemm_tile_heights_agree(gpu, n, k, full):
     """At `full` rows the tiles are 128 high, below 64 (a remainder of 1 to 64 rows in the last one):
     a row's sums run in the same order, so the same bits."""
@@ -491,10 +491,24 @@ def test_q8_gemm_tile_heights_agree(gpu, n, k, full):
 @pytest.mark.parametrize("m", [300, 1024])
 @pytest.mark.parametrize("with_y", [True, False])
 def test_q8_gemm_large_q8_out(gpu, n, k, m, with_y):
-    """The 128 x 128 GEMM (above 256 rows) with bias + ReLU: the fp32 rows within 2e-6 of the
-    oracle's scale, the Q8_0 rows the x86 quantisation of those fp32 rows bit for bit, rows past m
-    untouched. Two epilogues: fp32 + Q8_0 (a block is 8 lanes of 4 columns) and Q8_0 alone (a
-    block is 2 lanes of 16 columns; its fp32 rows then come from a second call with fp32 only)."""
+    """The GEMM above 256 rows (at these, tiles of 64 rows) with bias + ReLU."""
+    _check_large_q8_out(gpu, n, k, m, with_y)
+
+
+@pytest.mark.parametrize("n,k,m", [(2048, 512, 8100), (1536, 512, 11000), (512, 2048, 32700), (4096, 1024, 1550),
+                                   (1024, 4096, 6100)])
+@pytest.mark.parametrize("with_y", [True, False])
+def test_q8_gemm_128_row_tiles_q8_out(gpu, n, k, m, with_y):
+    """The same where the tiles are 128 rows high, with a remainder of rows in the last one."""
+    assert n // 128 * ((m + 127) // 128) >= (1024 if k in (512, 2048) else 384) and m % 128
+    _check_large_q8_out(gpu, n, k, m, with_y, np.r_[0:70, 120:136, m // 2:m // 2 + 40, m - 140:m])
+
+
+def _check_large_q8_out(gpu, n, k, m, with_y, rows=slice(None)):
+    """The fp32 rows within 2e-6 of the oracle's scale (`rows` of them), the Q8_0 rows the x86 quantisation
+    of those fp32 rows bit for bit, rows past m untouched. Two epilogues: fp32 + Q8_0 (a block is 8 lanes
+    of 4 columns) and Q8_0 alone (a block is 2 lanes of 16 columns; its fp32 rows then come from a second
+    call with fp32 only)."""
     import torch
     rng = np.random.default_rng(7200 + n + k + m)
     W = rng.standard_normal((n, k)).astype(np.float32) * 0.02
@@ -520,8 +534,8 @@ def test_q8_gemm_large_q8_out(gpu, n, k, m, with_y):
     y, yq, yd = y.cpu().numpy(), yq.cpu().numpy(), yd.cpu().numpy()
     assert (y[m] == 7.0).all() and (yq[m] == 5).all() and (yd[m] == 3.0).all()
     y, yq, yd = y[:m], yq[:m], yd[:m]
-    ref = np.maximum(O.q8_matmul(wb, n, k, X) + b[None, :], 0.0)
-    assert np.abs(y - ref).max() <= 2e-6 * np.abs(ref).max()
+    ref = np.maximum(O.q8_matmul(wb, n, k, X[rows]) + b[None, :], 0.0)
+    assert np.abs(y[rows] - ref).max() <= 2e-6 * np.abs(ref).max()
     assert (yd[1, 0] == 0.0) and (yq[1, :32] == 0).all()
     q_ref, d_ref = blocks_to_split(O.q8_quantize_x86(y), m, n)
     assert np.array_equal(yq, q_ref.reshape(m, n))
