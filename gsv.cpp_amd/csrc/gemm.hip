@@ -437,6 +437,21 @@ __global__ void __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu
     gemm_epilogue<MT>(sm.y, acc, 0.5f, out, n, m, n0, m0, wave, lane);   // (acc holds twice the output)
 }
 
+// Whether k_q8_gemm takes 64-row tiles, given the number of 128-row ones: twice the workgroups, three
+// instead of two of them resident on a CU. Up to 384 that is one round of at most 768; from 385 to 512 it
+// is two where 128-row tiles need one, which costs at K 1024 and above; further up by measurement. us,
+// 64-row / 128-row tiles (number of the latter):
+//   K 2048, N  512: 300 rows (12) 19.4 / 30.9, 6411 (204) 31.9 / 35.6, 12288 (384) 44.2 / 54.0, 12289 (388) 55.8 / 53.7,
+//                   14000 (440) 56.0 / 54.1, 16384 (512) 56.5 / 56.3, 16385 (516) 66.2 / 79.2, 25600 (800) 94.6 / 100.4
+//   K  512, N  512: 300 rows (12)  9.0 / 12.0, 6411 (204) 12.7 / 13.8, 16384 (512) 21.0 / 21.4, 25600 (800) 32.3 / 36.2
+//   K  512, N 2048: 300 rows (48)  8.6 / 11.6, 6411 (816) 32.4 / 34.1, 10000 (1264) 44.7 / 42.7, 25600 (3200) 100.2 / 99.1
+//   K 1024, N 4096: 600 rows (160) 19.0 / 20.9, 1536 (384) 26.0 / 31.5, 1537 (416) 32.4 / 31.7, 4000 (1024) 65.4 / 61.9
+//   K 4096, N 1024: 600 rows (40) 36.7 / 60.1, 4000 (256) 60.1 / 71.6, 6144 (384) 81.7 / 102.2, 6145 (392) 105.3 / 99.8
+// (the rows of N 1024 and 4096 are the BERT encoder's)
+constexpr bool gemm_half_tiles(int64_t k, int64_t tiles) {
+    return tiles <= 384 || (k == 512 && tiles < 1024) || (k == 2048 && tiles > 512 && tiles < 1024);
+}
+
 // ---- Q8_0 activations x fp16 weights on the fp16 matrix cores (the prefill's fp16 mode) ----
 // The tiling, staging and epilogue of k_q8_gemm, for weights dequantised once to fp16
 // (w16[n][k] = fp16(d * q), nearest even) and activations still in Q8_0: each wave turns its A
@@ -700,15 +715,6 @@ int launch_q8h_gemm(const uint16_t * w16, int64_t n, int64_t k, int64_t m, const
 // (lane (li, lg): 16 values of row/column li, half lg of the block), a group of blocks ahead of
 // its use. The four partial tiles are summed through LDS in wave order, so the result does not
 // depend on timing. Same arithmetic per block as k_q8_gemm.
-// Number of 128-row tiles below which k_q8_gemm takes 64-row ones: twice the workgroups, three
-// instead of two of them resident on a CU. us, 64-row / 128-row tiles (number of the latter):
-//   K 2048, N  512: 300 rows (12) 19.4 / 30.9, 6411 (204) 31.9 / 35.6, 16384 (512) 57.2 / 57.3, 25600 (800) 94.6 / 100.4
-//   K  512, N  512: 300 rows (12)  9.0 / 12.0, 6411 (204) 12.7 / 13.8, 16384 (512) 21.0 / 21.4, 25600 (800) 32.3 / 36.2
-//   K  512, N 2048: 300 rows (48)  8.6 / 11.6, 6411 (816) 32.4 / 34.1, 10000 (1264) 44.7 / 42.7, 25600 (3200) 100.2 / 99.1
-//   K 1024, N 4096: 600 rows (160) 19.0 / 20.9, 2000 (512) 34.1 / 33.6, 4000 (1024) 65.4 / 61.9
-//   K 4096, N 1024: 600 rows (40) 36.7 / 60.1, 4000 (256) 60.1 / 71.6, 6411 (408) 103.4 / 100.5, 8192 (512) 111.6 / 106.0
-// (the rows of N 1024 and 4096 are the BERT encoder's)
-constexpr int64_t gemm_half_tiles(int64_t k) { return k == 512 || k == 2048 ? 1024 : 384; }
 constexpr int64_t GS_MAX_ROWS = 256;      // launch_q8_gemm takes this kernel up to this many rows
 
 template <int NBLK, int MT, int W = 4>   // W waves, each a W-th of K
@@ -942,7 +948,7 @@ int launch_q8_gemm(const Q8Weights & w, int64_t n, int64_t k, int64_t m, const i
                  "q8_gemm: above %lld rows the operands are in natural order", (long long) GS_MAX_ROWS);
     const int8_t * ws = w.qn;
     const uint16_t * wd = w.dn;
-    const bool half = n / GM_BN * ((m + GM_BM - 1) / GM_BM) < gemm_half_tiles(k);
+    const bool half = gemm_half_tiles(k, n / GM_BN * ((m + GM_BM - 1) / GM_BM));
     const int64_t bm = half ? GM_BM / 2 : GM_BM;
     const dim3 grid((unsigned) (n / GM_BN * ((m + bm - 1) / bm)));
 #define GSVK_GM(NB)                                                                                                \
