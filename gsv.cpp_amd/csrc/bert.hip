@@ -231,8 +231,9 @@ __global__ void __launch_bounds__(256) k_bert_attn(const float * __restrict__ qk
 //     K slot (c, g) of the product holds the keys 16 c + 4 g + [0, 4) and 16 c + 8 + 4 g + [0, 4), and
 //     V^T is staged in that order. A tile's sum starts at zero (its small products first) and joins
 //     the running one in one fma with the rescaling.
-// It is bound by its instructions per tile (splits and softmax on the vector ALUs beside 48 products):
-// 16 sequences of 5 to 301 tokens 64.4 -> 33.2 us per layer, 8 of 33 to 97 16.7 -> 15.8.
+// It is bound by its instructions per tile (splits and softmax on the vector ALUs beside 48 products;
+// matrix cores busy 0.27 of the CUs' time): 16 sequences of 5 to 301 tokens 64.4 -> 33.2 us per layer, 8 of
+// 33 to 97 (128 workgroups) 15.1 -> 13.2 with fp16 output and 16.4 -> 15.6 with planes.
 // LDS: K chunk (step s of 16 dims, plane): slot 32 g + (key ^ (2 s + g)), so that the 8 threads that
 // write a key's 8 dim groups hit different banks; V^T chunk (dim tile, c, plane): slot 32 g + dim % 32.
 constexpr int BM_Q = 128;   // queries per workgroup
@@ -487,7 +488,7 @@ __global__ void __launch_bounds__(BG_WAVES * 64) k_bert_gemm(const T * __restric
     const int li = lane & 31, lg = lane >> 5;
     const int n0 = blockIdx.x * BG_BN, m0 = blockIdx.y * BM, p = blockIdx.z;
     const int kw = kslice / BG_WAVES;
-    // fp16 operands in the operand order (bt_off; rows padded to 64): a step of the wave is one
+    // fp16 operands in the operand order (bt_off; rows padded to BG_ROW_PAD): a step of the wave is one
     // 1 KB chunk at stride SSTEP; fp32 operands row-major, the lane at its row and slot
     constexpr bool TL = sizeof(T) == 2;
     constexpr int64_t SSTEP = TL ? 512 : St::K;
@@ -873,13 +874,17 @@ int load_ln(gsvk_bert * m, const GgufFile & g, const std::string & wn, const std
 }
 
 // Rows above which the LDS-tiled GEMM takes the projections; at most these the direct loads, which
-// put every weight's load in flight at once. Whole encode of one sequence, us, direct / tiled:
-//   F16  64 rows 825 / 1316, 256 rows 1403 / 1750, 384 rows 1870 / 2060, 512 rows 2105 / 2215;
-//        of several: 2 x 257 rows 2107 / 2038, 6 x 120 2102 / 2135, 8 x 128 2419 / 2494,
-//        3 x 290 2515 / 2448, 4 x 300 3049 / 2868, 16 x 128 3895 / 3539
-//   F32  64 rows 1257 / 1702, 96 rows 1836 / 1792, 128 rows 1855 / 1834, 160 rows 2845 / 2055,
-//        512 rows 5103 / 3425
-// (the F16 lines run together from 512 to 1024 rows and part above; the F32 lines meet near 90)
+// put every weight's load in flight at once. Whole encode, us, direct / tiled:
+//   F16  one sequence: 64 rows 825 / 1316, 256 rows 1403 / 1750, 384 rows 1870 / 2060, 512 rows 2110 / 2224;
+//        9 x 64 rows 1865 / 1834, 2 x 320 2244 / 2174, 2 x 330 2357 / 2414, 6 x 120 2129 / 2145,
+//        12 x 64 2105 / 2105, 2 x 400 2614 / 2552, 14 x 64 2299 / 2201, 15 x 64 2375 / 2373,
+//        8 x 128 2464 / 2501, 15 x 70 2710 / 2580, 4 x 300 3112 / 2889, 24 x 64 3189 / 2927
+//   F32  64 rows 1257 / 1702, 80 rows 1756 / 1770, 96 rows 1842 / 1804, 128 rows 1849 / 1849,
+//        130 rows 2691 / 2035, 160 rows 2848 / 2073, 512 rows 5103 / 3425
+// F16: at 512 rows the direct loads are 5 % faster. Both go in steps of 64 rows, of unlike height (the
+// tiled QKV has more than a workgroup per CU from 641 rows, its FFN1 takes 128-row tiles from 897), and
+// cross several times up to 1024 rows: tiled 4 % faster to 2 % slower, 1 % faster on the whole, and
+// always faster above. F32: the two meet between 90 and 128 rows and part from 129.
 constexpr int64_t BERT_DIRECT_ROWS_F16 = 512;
 constexpr int64_t BERT_DIRECT_ROWS_F32 = 96;
 bool bert_lds(const Proj & w, int64_t M) { return M > (w.f16 ? BERT_DIRECT_ROWS_F16 : BERT_DIRECT_ROWS_F32); }
@@ -911,8 +916,10 @@ int launch_bert_lds(gsvk_bert * m, const uint16_t * X, const uint16_t * W, int64
 // Workgroups of the matrix-core attention (128 queries of a sequence and head each) above which it is
 // taken: with fewer the lane-per-query kernel's 8 times as many workgroups fill the chip better. Whole
 // encode of an F16 file, us, lane per query / matrix cores: 1 x 256 tokens (32 workgroups) 1406 / 1465,
-// 1 x 512, 2 x 256 and 4 x 64 (64) 2131 / 2142, 1817 / 1822 and 1215 / 1217, 8 x 32 and 8 x 64 (128)
-// 1203 / 1166 and 1617 / 1571, 16 x 200 (512) 6564 / 5104.
+// 1 x 512, 2 x 256 and 4 x 64 (64) 2131 / 2142, 1817 / 1822 and 1215 / 1217, 5 x 64 and 5 x 100 (80) 1417 /
+// 1414 and 1719 / 1677, 8 x 32 and 8 x 64 (128) 1186 / 1166 and 1605 / 1597, 16 x 200 (512) 6564 / 5104. Of an
+// F32 file (three planes to write): 4 x 64 2093 / 2130, 5 x 64 2487 / 2493, 5 x 100 3035 / 3024, 8 x 64 2948 /
+// 2954, 8 x 128 (128) 4971 / 4773.
 constexpr int BERT_ATTN_WGS = 64;
 
 // Row tiles of 32 per wave: 2 (64-row workgroups) when that still gives 256 workgroups, else 1.
@@ -1152,7 +1159,8 @@ extern "C" int gsvk_bert_encode(gsvk_bert * m, int B, const int32_t * ids_flat, 
     DevGuard guard(m->device);
     hipStream_t st = m->stream;
     // workspace: x, qkv, attention output, projection output (up to BERT_MAX_SLICES partial
-    // rows), FFN hidden, the fp16 GEMM inputs (a D-wide row, the FFN hidden), the small arrays
+    // rows), FFN hidden, the GEMM inputs (a D-wide row, the FFN hidden) as fp16, as planes and as
+    // Q8_0 rows with their scales, the small arrays
     const size_t fl = (size_t) rows * (D + 3 * D + D + (size_t) BERT_MAX_SLICES * D + F);
     const int64_t rowsp = (rows + BG_ROW_PAD - 1) / BG_ROW_PAD * BG_ROW_PAD;   // rows of the operand order
     const size_t n16 = m->any_f16 ? (size_t) rowsp * (D + F) : 0;

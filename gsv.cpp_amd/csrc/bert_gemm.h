@@ -6,8 +6,10 @@
 // [8 g, 8 g + 8) of the step. PL = 1: fp16 values (F16 weights and the activations that meet them,
 // as ggml-cpu rounds them). PL = 3: fp32 values as three bf16 planes x = h + m + l, exact (each
 // takes 8 of the 24 significant bits; bf16 has the range of fp32), so that an F32 product
-//   x * w = hh + (hm + mh) + (mm + hl + lh)      (ml, lm, ll: below 2^-26 of the product)
-// is six v_mfma_f32_32x32x16_bf16 with fp32 accumulation. The five small ones have accumulators of
+//   x * w = hh + (hm + mh) + (mm + hl + lh)
+// is six v_mfma_f32_32x32x16_bf16 with fp32 accumulation. What is left out, ml + lm + ll, is at
+// most 2^-24 of the product (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|), the size of one fp32 rounding of it, and
+// 2^-27.5 of it rms (values uniform in [1, 2)). The five small products have accumulators of
 // their own, so the large sum is rounded once per 16 K values; the fp32 matrix instruction rounds
 // once per 2. The bf16 matrix cores run 16 times as fast as the fp32 ones, six products 2.7 times.
 #pragma once
@@ -119,12 +121,13 @@ __device__ __forceinline__ void bg_load_lds(const uint16_t * base, uint32_t off,
 
 // Y[M][N] (or a K slice of it) = X[M][K] . W[N][K]^T. Workgroup: WM x WN waves, each TM x TN MFMA
 // tiles of 32 x 32; K streams through LDS in stages of KS steps by direct global -> LDS loads,
-// NBUF buffers deep, one barrier per stage. Before, 64 x 32 tiles without sharing read 0.9 GB through
+// NBUF buffers deep (NBUF - 1 stages in flight), one barrier per stage. Before, 64 x 32 tiles without sharing read 0.9 GB through
 // the L2 per FFN1 of 2265 rows; 128 x 128 tiles read 0.3 GB. Measured (fp32 output, us, before -> now):
 // fp16 2265 rows N 4096 K 1024 52 -> 32, N 1024 K 4096 49 -> 36; planes 564 rows N 4096 K 1024 79 -> 34,
-// N 1024 K 4096 95 -> 33. The products alone (no loads, no reads) take 23 of the 32 us and 23 of the
-// 34, the loads alone 27 and 27: what is left is their overlap and the stores. A chunk is one load instruction of a wave and one
-// conflict-free 16-byte read per lane. The weights are the MFMA's A operand, so a lane holds 4
+// N 1024 K 4096 95 -> 33. The matrix cores are busy for 0.22 to 0.31 (fp16) and 0.43 (planes) of the CUs'
+// time, the waves wait for a third to half of theirs (counters): the loads and their overlap bound it, not
+// the products. A chunk is one load instruction of a wave and one conflict-free 16-byte read per lane
+// (SQ_LDS_BANK_CONFLICT 0). The weights are the MFMA's A operand, so a lane holds 4
 // consecutive columns of one row per register quad and the epilogue stores from registers.
 template <int PL, int TM, int TN, int WM, int WN, int KS, int NBUF>
 __global__ void __launch_bounds__(WM * WN * 64) k_bert_gemm_lds(const uint16_t * __restrict__ X,

@@ -191,7 +191,7 @@ __device__ __forceinline__ void q8_store_natural(int8_t * row, int blk, int sub,
 // Layouts of a Q8_0 matrix [rows][k] whose scales are stored apart from the quants:
 //   Q8_SLICED  quants of row r: group j of every block together, qs[r][j][blk][4] (the GEMV's
 //              operand), scales [r][k/32];
-//   Q8_NATURAL quants [r][k] in order, scales [r][k/32] (the 128 x 128 GEMM's operand);
+//   Q8_NATURAL quants [r][k] in order, scales [r][k/32] (the LDS-tiled GEMM's operand);
 //   Q8_TILED   the matrix-core operand order of the small-batch GEMM: for each 32-row tile and
 //              block, 1 KB in which lane L = 32*h + i holds the 16 quants [16h, 16h+16) of
 //              row i of the tile at bytes [16L, 16L+16); scales per (tile, block) as 32

@@ -57,7 +57,7 @@ struct LayerOut {
     int rows_per_seq;
     const int32_t * col_ptr;
     int col_add;
-    // (128 x 128 GEMM only) left-padding rows per sequence of rows_per_seq rows: a row tile that
+    // (GEMM above 256 rows only) left-padding rows per sequence of rows_per_seq rows: a row tile that
     // holds only padding rows writes zeros to y / yq / yd and skips its products and K/V (no
     // query attends a padding key), or null
     const int32_t * row_pad;
@@ -75,11 +75,11 @@ struct Q8Weights {
 
 // Q8_0 x Q8_0 GEMM on the matrix cores (gemm.hip) with the same epilogue options: n % 32 == 0,
 // k in {512, 1024, 2048, 4096} (1024 and 4096: the BERT encoder's Q8_0 projections). Activations
-// xs [m][k] with fp32 scales xd [m][k/32] (fp16 values) in x_layout: Q8_NATURAL, or Q8_TILED (rows padded to 32; small-batch kernel only); a Q8_0 output
-// is written in out.yq_layout (Q8_NATURAL or Q8_TILED). Up to 256 rows (or n % 128 != 0) a kernel
-// of 32-column tiles runs (tiled weights if given), tile_rows (1, 2 or 4 row tiles of 32 per
-// workgroup, 0 = its own choice) selecting its row tiling; above, the 128 x 128 kernel (natural
-// operands only).
+// xs [m][k] with fp32 scales xd [m][k/32] (fp16 values) in x_layout: Q8_NATURAL, or Q8_TILED (rows
+// padded to 32; small-batch kernel only); a Q8_0 output is written in out.yq_layout (Q8_NATURAL or
+// Q8_TILED). Up to 256 rows (or n % 128 != 0) a kernel of 32-column tiles runs (tiled weights if given),
+// tile_rows (1, 2 or 4 row tiles of 32 per workgroup, 0 = its own choice) selecting its row tiling;
+// above, the LDS-tiled kernel of 64 or 128 rows x 128 columns (natural operands only).
 int launch_q8_gemm(const Q8Weights & w, int64_t n, int64_t k, int64_t m, const int8_t * xs,
                    const float * xd, int x_layout, const LayerOut & out, hipStream_t stream,
                    int tile_rows = 0);
@@ -90,7 +90,7 @@ int launch_q8_dequant_f16(const int8_t * q, const uint16_t * d, int64_t n, int64
 
 // The same projection on the fp16 matrix cores (gemm.hip): the Q8_0 activations (natural order)
 // taken as fp16(d * q) times the fp16 weights w16 [n][k] of launch_q8_dequant_f16, fp32
-// accumulation, the epilogue of launch_q8_gemm's 128 x 128 kernel (natural-order Q8_0 output);
+// accumulation, the epilogue of launch_q8_gemm's LDS-tiled kernel (natural-order Q8_0 output);
 // n % 128 == 0, k 512 or 2048.
 int launch_q8h_gemm(const uint16_t * w16, int64_t n, int64_t k, int64_t m, const int8_t * xs, const float * xd,
                     const LayerOut & out, hipStream_t stream);
